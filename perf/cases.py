@@ -1,0 +1,636 @@
+"""The work that users of this package have it do, as cases that can be timed and compared.
+
+A case is one run of a simulation (or of many at once) the way a program does it: the
+initial state goes in, the time loop advances it, the updated fields come back to the host.
+Kinds of case, and what each stands for:
+
+  tube      1-D hydro shock tube (Sod and its relatives), transparent ends
+  vortex    2-D ideal MHD on a periodic box (Orszag-Tang), constrained transport
+  shear     2-D hydro shear layer (Kelvin-Helmholtz), circular x / constant y
+  blast     3-D hydro blast wave (Sedov), transparent boundaries
+  mhd3d     3-D ideal MHD on a periodic box
+  source    3-D hydro with a fixed gravitational potential, radiation and artificial viscosity
+  ensemble  many 1-D MHD Riemann problems and shear layers advanced together (FP32 bulk)
+  serve     a queue of solve requests under continuous batching (FP32 bulk)
+
+Precision "fp64" is the plain path and "fp32" the FP32-bulk path, whose fields hold FP32
+values (they are returned as such).  "sweep" is the fluid sweep setting of the run.
+"""
+import math
+
+import numpy as np
+import torch
+
+from imogen_amd import autotune, create_arrays, initialize, problems
+from imogen_amd.ensemble import Ensemble
+from imogen_amd.serve import DONE, FAILED, Server
+
+FLUID = ["mass", "momx", "momy", "momz", "ener"]
+MAGNET = ["magx", "magy", "magz"]
+FOREVER = 10 ** 8  # iterMax of runs whose length the program chooses
+
+
+def listed():
+    return [
+        # the smallest call: a short 1-D tube, a few iterations (latency and launches)
+        {"name": "tube_fp32_257", "kind": "tube", "prec": "fp32", "nx": 257, "limiter": "superbee",
+         "iterations": 24},
+        # the Sod tube of the configurations: 1024 cells, 200 iterations
+        {"name": "tube_fp64_1024", "kind": "tube", "prec": "fp64", "nx": 1024,
+         "limiter": "vanleer", "iterations": 200},
+        # Orszag-Tang 512^2 (the 2-D MHD configuration), plain path
+        {"name": "vortex_fp64_512", "kind": "vortex", "prec": "fp64", "n": 512,
+         "limiter": "superbee", "iterations": 240},
+        # a small, odd MHD box in FP32
+        {"name": "vortex_fp32_191", "kind": "vortex", "prec": "fp32", "n": 191,
+         "limiter": "vanleer", "iterations": 120},
+        # shear layers: one of the ensemble's largest boxes alone in FP32, a ragged one in FP64
+        {"name": "shear_fp32_1024", "kind": "shear", "prec": "fp32", "n": 1024,
+         "limiter": "vanleer", "iterations": 200},
+        {"name": "shear_fp64_333", "kind": "shear", "prec": "fp64", "n": 333,
+         "limiter": "vanleer", "iterations": 150},
+        # Sedov 256^3 (the 3-D configuration) on the plain path's sweep for large grids
+        {"name": "blast_fp64_256", "kind": "blast", "prec": "fp64", "n": 256,
+         "limiter": "minmond", "sweep": "auto_fast", "iterations": 120},
+        # the same problem on an odd grid with the default sweep, and in FP32
+        {"name": "blast_fp64_125", "kind": "blast", "prec": "fp64", "n": 125,
+         "limiter": "vanleer", "sweep": "general", "iterations": 100},
+        {"name": "blast_fp32_192", "kind": "blast", "prec": "fp32", "n": 192,
+         "limiter": "minmond", "sweep": "general", "iterations": 150},
+        # 3-D MHD, ragged
+        {"name": "mhd3d_fp64_100", "kind": "mhd3d", "prec": "fp64", "nx": 100, "ny": 90, "nz": 75,
+         "limiter": "vanleer", "iterations": 60},
+        # every source term at once
+        {"name": "source_fp64_96", "kind": "source", "prec": "fp64", "nx": 96, "ny": 80,
+         "nz": 64, "limiter": "vanleer", "iterations": 80},
+        # a quarter of the benchmark's ensemble between two outputs of the fields
+        {"name": "ensemble_fp32", "kind": "ensemble", "prec": "fp32", "riemann": 128, "shear": 16,
+         "pick": 0, "iterations": 120},
+    ]
+
+
+def _odd_size(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    """Lengths grow with the grid (a fixed time in crossings of the box), as those of runs do."""
+    kind = rng.choice(["tube", "tube", "vortex", "vortex", "shear", "shear", "blast", "blast",
+                       "mhd3d", "source", "ensemble", "serve"])
+    prec = rng.choice(["fp64", "fp32"])
+    lim = rng.choice(["vanleer", "superbee", "minmond"])
+    if kind == "tube":
+        n = _odd_size(rng, 64, 4096)
+        return {"kind": kind, "prec": prec, "nx": n, "limiter": lim,
+                "iterations": min(200, max(16, n // 5))}
+    if kind == "vortex":
+        n = _odd_size(rng, 48, 640)
+        return {"kind": kind, "prec": prec, "n": n, "limiter": rng.choice(["vanleer", "superbee"]),
+                "iterations": min(120, n // 2)}
+    if kind == "shear":
+        n = _odd_size(rng, 64, 1024)
+        return {"kind": kind, "prec": prec, "n": n, "limiter": lim, "iterations": min(120, n // 3)}
+    if kind == "blast":
+        sweep = rng.choice(["general", "auto_fast"]) if prec == "fp64" else "general"
+        # the sweep for large grids takes power-of-two pencils: half of its draws are one
+        n = 128 if sweep == "auto_fast" and rng.random() < 0.5 else _odd_size(rng, 32, 200)
+        return {"kind": kind, "prec": prec, "n": n, "limiter": lim, "sweep": sweep,
+                "iterations": min(60, n // 2)}
+    if kind in ("mhd3d", "source"):
+        n = [_odd_size(rng, 24, hi) for hi in (128, 128, 96)]
+        return {"kind": kind, "prec": prec, "nx": n[0], "ny": n[1], "nz": n[2],
+                "limiter": "vanleer", "iterations": min(50, min(n) // 2)}
+    if kind == "ensemble":
+        return {"kind": kind, "prec": "fp32", "riemann": rng.randint(8, 96),
+                "shear": rng.randint(1, 10), "pick": rng.randint(1, 10 ** 6),
+                "iterations": rng.randint(48, 96)}
+    return {"kind": kind, "prec": "fp32", "size": _odd_size(rng, 96, 256),
+            "requests": rng.randint(4, 10), "iterations": 0}
+
+
+# ---- initial states ---------------------------------------------------------------------
+
+def _tube(case, rng):
+    """A Sod-like tube: two states at rest, the left one denser and at higher pressure."""
+    n = case["nx"]
+    ini, st = problems.sod(n, limiter=case["limiter"], iter_max=FOREVER)
+    right = st["mass"] < 0.5
+    gm1 = ini["gamma"] - 1.0
+    st["mass"] = np.where(right, rng.uniform(0.1, 0.2), rng.uniform(0.8, 1.2))
+    st["ener"] = np.where(right, rng.uniform(0.08, 0.12), rng.uniform(0.8, 1.2)) / gm1
+    return ini, st
+
+
+def _vortex(case, rng):
+    """Orszag-Tang with the amplitudes of its velocity and field varied."""
+    ini, st = problems.orszag_tang(case["n"], limiter=case["limiter"], iter_max=FOREVER)
+    a, b = rng.uniform(0.9, 1.1), rng.uniform(0.9, 1.1)
+    rho, gm1 = st["mass"], ini["gamma"] - 1.0
+    st["mom"] = [a * m for m in st["mom"]]
+    st["mag"] = [b * m for m in st["mag"]]
+    st["ener"] = (5.0 / (12.0 * math.pi) / gm1 + 0.5 * sum(m * m for m in st["mom"]) / rho
+                  + 0.5 * sum(m * m for m in st["mag"]))
+    return ini, st
+
+
+def _axes(nx, ny, nz):
+    return (2.0 * math.pi * np.arange(nx)[None, None, :] / nx,
+            2.0 * math.pi * np.arange(ny)[None, :, None] / ny,
+            2.0 * math.pi * np.arange(nz)[:, None, None] / nz)
+
+
+def _mhd3d(case, rng):
+    """A smooth magnetised flow on a periodic box; no component of B varies along itself."""
+    nx, ny, nz = case["nx"], case["ny"], case["nz"]
+    x, y, z = _axes(nx, ny, nz)
+    ph = rng.uniform(0.0, 2.0 * math.pi, 8)
+    full = np.zeros((nz, ny, nx))
+    ini, _ = problems.orszag_tang(4, limiter=case["limiter"], iter_max=FOREVER)
+    ini["grid"] = (nx, ny, nz)
+    ini["dGrid"] = tuple(2.0 * math.pi / n for n in (nx, ny, nz))
+    mass = 1.0 + 0.2 * np.sin(x + ph[0]) * np.cos(y + z + ph[1]) + full
+    vel = [0.5 * np.sin(y + ph[2]) + full, 0.5 * np.sin(z + ph[3]) + full,
+           0.5 * np.sin(x + ph[4]) + full]
+    mag = [0.4 * np.sin(z + ph[5]) + full, 0.4 * np.sin(2.0 * x + ph[6]) + full,
+           0.4 * np.sin(y + ph[7]) + full]
+    ener = (1.0 / (ini["gamma"] - 1.0) + 0.5 * mass * sum(v * v for v in vel)
+            + 0.5 * sum(b * b for b in mag))
+    return ini, {"mass": mass, "mom": [mass * v for v in vel], "ener": ener, "mag": mag}
+
+
+def _source(case, rng):
+    """A stratified, gently stirred layer; also the potential and the source settings."""
+    nx, ny, nz = case["nx"], case["ny"], case["nz"]
+    x, y, _ = _axes(nx, ny, nz)
+    z = (np.arange(nz)[:, None, None] + 0.5) / nz
+    ph = rng.uniform(0.0, 2.0 * math.pi, 3)
+    full = np.zeros((nz, ny, nx))
+    ini, _ = problems.sod(4, limiter=case["limiter"], iter_max=FOREVER)
+    ini["grid"] = (nx, ny, nz)
+    ini["dGrid"] = (1.0 / nx, 1.0 / ny, 1.0 / nz)
+    ini["bcMode"] = {"x": "circ", "y": "circ", "z": "const"}
+    mass = np.exp(-0.5 * z) * (1.0 + 0.1 * np.sin(x + ph[0]) * np.sin(y + ph[1])) + full
+    vel = [0.2 * np.sin(y + ph[2]) + full, 0.2 * np.cos(x + ph[0]) + full,
+           0.1 * np.sin(x + y + ph[1]) + full]
+    ener = np.exp(-0.5 * z) / (ini["gamma"] - 1.0) + 0.5 * mass * sum(v * v for v in vel)
+    st = {"mass": mass, "mom": [mass * v for v in vel], "ener": ener,
+          "mag": [np.zeros_like(full) for _ in range(3)]}
+    phi = 0.5 * z + 0.05 * np.sin(x + ph[2]) + full
+    return ini, st, {"potential": phi, "threshold": 0.05, "exponent": 0.5, "maximum": 0.5,
+                     "linear": 0.1, "quadratic": 1.0}
+
+
+def _shear(case, rng):
+    ini, _ = problems.kelvin_helmholtz(4, limiter=case["limiter"], iter_max=FOREVER)
+    ini = problems.resize(ini, (case["n"], case["n"], 1))
+    return ini, (float(rng.uniform(0.4, 0.6)), 8.0, 0.2, int(rng.integers(1 << 30)))
+
+
+def _blast(case, rng):
+    ini, _ = problems.sedov(4, limiter=case["limiter"], time_max=1e9, iter_max=FOREVER)
+    n = case["n"]
+    return problems.resize(ini, (n, n, n)), (3.0, 1e-5, float(rng.uniform(0.8, 1.2)))
+
+
+# sizes of the ensemble's and the queue's simulations: those of the benchmark, from `pick`
+# so that a seed changes the states and not the work
+def _ensemble(case, rng):
+    pick = np.random.default_rng(case["pick"])
+    sims = [problems.mhd_riemann(int(pick.integers(256, 4097)), seed=int(rng.integers(1 << 30)),
+                                 iter_max=FOREVER) for _ in range(case["riemann"])]
+    for _ in range(case["shear"]):
+        sims.append(problems.kelvin_helmholtz(int(pick.choice([128, 192, 256, 384, 512])),
+                                              seed=int(rng.integers(1 << 30)), iter_max=FOREVER))
+    return sims
+
+
+def _requests(case, rng):
+    out = []
+    for i in range(case["requests"]):
+        n = max(24, case["size"] * (4 - i % 3) // 4)
+        kind = ["kelvin_helmholtz", "orszag_tang", "sedov", "sod"][i % 4]
+        gamma = float(rng.uniform(1.4, 1.67))
+        if kind == "sedov":
+            n = max(16, n // 4)
+            ini, _ = problems.sedov(1, gamma=gamma, time_max=5e-3, iter_max=FOREVER)
+            dims, params = (n, n, n), (3.0, 1e-5, 1.0)
+        elif kind == "sod":
+            ini, _ = problems.sod(1, ny=1, bc="const", gamma=gamma, iter_max=FOREVER, time_max=0.2)
+            dims, params = (n, n, 1), ()
+        elif kind == "orszag_tang":
+            ini, _ = problems.orszag_tang(1, gamma=gamma, iter_max=FOREVER)
+            ini["timeMax"] = 0.5
+            dims, params = (n, n, 1), ()
+        else:
+            ini, _ = problems.kelvin_helmholtz(1, gamma=gamma, iter_max=FOREVER)
+            ini["timeMax"] = 0.2
+            dims, params = (n, n, 1), (0.5, 8.0, 0.01, int(rng.integers(1 << 30)))
+        out.append((problems.resize(ini, dims), kind, params))
+    return out
+
+
+# ---- prepare / run ----------------------------------------------------------------------
+
+HOST_STATES = {"tube": _tube, "vortex": _vortex, "mhd3d": _mhd3d, "source": _source}
+DEVICE_STATES = {"shear": (_shear, "kelvin_helmholtz"), "blast": (_blast, "sedov")}
+
+
+def prepare(case, seed):
+    rng = np.random.default_rng(seed)
+    kind, s = case["kind"], {"case": case}
+    if kind == "ensemble":
+        sims = _ensemble(case, rng)
+        s["ens"] = Ensemble(sims, "fp32")
+        autotune.apply(s["ens"], sims, autotune.load_table(), "fp32")
+        s["fields"] = [FLUID + (MAGNET if ini["mode"]["magnet"] else []) for ini, _ in sims]
+        return s
+    if kind == "serve":
+        s["server"], s["requests"] = Server("fp32", max_active=64), _requests(case, rng)
+        return s
+    if kind in DEVICE_STATES:
+        make, s["ic"] = DEVICE_STATES[kind]
+        ini, s["params"] = make(case, rng)
+    else:
+        ini, s["state"], *extra = HOST_STATES[kind](case, rng)
+    run = s["run"] = initialize(ini, case["prec"])
+    if "sweep" in case:
+        run.set_fluid_kernel(case["sweep"])
+    if kind == "source":
+        x = extra[0]
+        create_arrays(run, s["state"])  # the radiation's strength follows from the state
+        run.set_gravity(x["potential"], x["threshold"])
+        run.set_radiation("optically_thin", x["exponent"], x["maximum"])
+        run.set_viscosity("neumann_richtmyer", x["linear"], x["quadratic"])
+    return s
+
+
+def run(s):
+    """One pass.  A single simulation starts from its initial state on every pass; an
+    ensemble goes on from where the last output left it."""
+    case = s["case"]
+    kind = case["kind"]
+    if kind == "ensemble":
+        ens = s["ens"]
+        ens.step(case["iterations"])
+        out = {f: [] for f in FLUID + MAGNET}
+        for i, fields in enumerate(s["fields"]):
+            for f in fields:
+                out[f].append(ens.download(i, f).astype(np.float32).ravel())
+        return {f: np.concatenate(v) for f, v in out.items()}
+    if kind == "serve":
+        srv, out = s["server"], {}
+        ids = {srv.submit_problem(ini, ic, params): i
+               for i, (ini, ic, params) in enumerate(s["requests"])}
+        pending = set(ids)
+        while pending:
+            srv.step(4)
+            for rid in sorted(pending):
+                status = srv.status(rid)[0]
+                if status == FAILED:
+                    raise RuntimeError("request %d failed" % ids[rid])
+                if status == DONE:
+                    fields = _fields(s["requests"][ids[rid]][0])
+                    out["r%d" % ids[rid]] = np.stack(
+                        [srv.download(rid, f).astype(np.float32) for f in fields])
+                    srv.release(rid)
+                    pending.discard(rid)
+        return out
+    sim = s["run"]
+    if "ic" in s:
+        sim.init_problem(s["ic"], s["params"])
+    else:
+        create_arrays(sim, s["state"])
+    sim.run_iterations(case["iterations"])
+    dtype = np.float64 if case["prec"] == "fp64" else np.float32
+    fields = FLUID + (MAGNET if sim.magnet.ACTIVE else [])
+    return {f: sim.download(f).astype(dtype, copy=False) for f in fields}
+
+
+def _fields(ini):
+    return FLUID + (MAGNET if ini["mode"]["magnet"] else [])
+
+
+# ---- work -------------------------------------------------------------------------------
+
+def _dims(case):
+    k = case["kind"]
+    if k == "tube":
+        return (case["nx"], 1, 1), False
+    if k in ("vortex", "shear"):
+        return (case["n"], case["n"], 1), k == "vortex"
+    if k == "blast":
+        return (case["n"],) * 3, False
+    return (case["nx"], case["ny"], case["nz"]), k == "mhd3d"
+
+
+def _step_work(dims, mhd, esz, iterations):
+    """Bytes and operations of `iterations` iterations of one simulation.  A sweep needs the
+    largest signal speed of each whole pencil before it can update a cell, so a grid is
+    read and written once per sweep; a 1-D run's single pencil once per run."""
+    cells = dims[0] * dims[1] * dims[2]
+    sweeps = 2 * sum(n >= 3 for n in dims) * iterations
+    fields = 8 if mhd else 5
+    passes = 1 if dims[1] == dims[2] == 1 else sweeps
+    return {"bytes": 2.0 * fields * esz * cells * passes,
+            "flops": (440.0 if mhd else 250.0) * cells * sweeps}
+
+
+def work(case):
+    esz = 8 if case["prec"] == "fp64" else 4
+    if case["kind"] == "ensemble":
+        parts = [(ini["grid"], ini["mode"]["magnet"], case["iterations"])
+                 for ini, _ in _ensemble(case, np.random.default_rng(0))]
+    elif case["kind"] == "serve":
+        parts = []
+        for ini, _, _ in _requests(case, np.random.default_rng(0)):
+            # two time steps of about CFL * dx / 2 per iteration
+            per = 2.0 * ini["cfl"] * ini["dGrid"][0] / 2.0
+            parts.append((ini["grid"], ini["mode"]["magnet"], max(1.0, ini["timeMax"] / per)))
+    else:
+        parts = [_dims(case) + (case["iterations"],)]
+    total = {"bytes": 0.0, "flops": 0.0}
+    for dims, mhd, its in parts:
+        w = _step_work(dims, mhd, esz, its)
+        for k in total:
+            total[k] += w[k]
+    return total
+
+
+# ---- the same runs in plain 64-bit torch ------------------------------------------------
+
+PERMS = [(3, 2, 1), (3, 1, 2), (2, 3, 1), (2, 1, 3), (1, 2, 3), (1, 3, 2)]
+FORWARD = {1: (2, 3), 2: (1, 3), 3: (1, 2)}
+
+
+class _Exact:
+    """Relaxing-TVD hydro and constrained-transport MHD on whole arrays of shape
+    (nz, ny, nx); one boundary mode per dimension: circ, const or trans (hydro)."""
+
+    def __init__(self, ini, st, sources=None):
+        bc, dev = ini["bcMode"], "cuda" if torch.cuda.is_available() else "cpu"
+        to = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device=dev)  # noqa: E731
+        self.n, self.dx = ini["grid"], ini["dGrid"]
+        self.ndims = 3 if self.n[2] > 1 else 2
+        self.bc = [bc] * 3 if isinstance(bc, str) else [bc[k] for k in "xyz"]
+        self.g, self.cfl, self.lim = ini["gamma"], ini["cfl"], ini["fluxLimiter"]
+        self.minmass, self.inf = ini["minMass"], float(ini["bcInfinity"])
+        self.mhd, self.time, self.time_max = ini["mode"]["magnet"], 0.0, ini["timeMax"]
+        self.q = [to(a) for a in (st["mass"], *st["mom"], st["ener"])]
+        self.b = [to(a) for a in st["mag"]] if self.mhd else None
+        self.edges, self.src = {}, sources
+        if self.mhd:
+            self.c = [0.5 * (self.b[k] + self.shift(self.b[k], k, 1)) for k in range(3)]
+        if sources:
+            self.phi, a = to(sources["potential"]), sources["exponent"]
+            q = self.q
+            ke = 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0]
+            unscaled = q[0] ** (2.0 - a) * self.gas() ** a
+            self.strength = sources["maximum"] / 100.0 * float(((q[4] - ke) / unscaled).min())
+
+    # shifts: position i of shift(a, d, m) holds a[i + m]
+    def shift(self, a, d, m, obj=None):
+        if d >= self.ndims:
+            return a
+        ax, n = 2 - d, a.shape[2 - d]
+        if self.bc[d] == "circ":
+            return torch.roll(a, -m, ax)
+        k = min(abs(m), n)
+        if self.bc[d] == "const" or obj is None:
+            end = a.narrow(ax, n - 1 if m > 0 else 0, 1)
+            ghost = torch.repeat_interleave(end, k, ax)
+        else:
+            ghost = self.open_end(a, d, m > 0, obj)
+        inner = a.narrow(ax, k if m > 0 else 0, n - k)
+        return torch.cat([inner, ghost] if m > 0 else [ghost, inner], ax)
+
+    def assign(self, obj, a):
+        """The first array an object holds gives its stored edges."""
+        if (obj, 0, 0) in self.edges:
+            return
+        for d in range(self.ndims):
+            ax = 2 - d
+            self.edges[obj, 0, d] = a.narrow(ax, 0, 1).clone()
+            self.edges[obj, 1, d] = a.narrow(ax, a.shape[ax] - 1, 1).clone()
+
+    def open_end(self, a, d, upper, obj):
+        """Transparent ghost: the shape-preserving cubic through the last three cells and
+        the stored edge at the distance bcInfinity, one cell out."""
+        ax = 2 - d
+        n = a.shape[ax]
+        at = [n - 3, n - 2, n - 1] if upper else [2, 1, 0]
+        y0, y1, y2 = (a.narrow(ax, min(max(i, 0), n - 1), 1) for i in at)
+        key = (obj, int(upper), d)
+        diff = y2 - self.edges[key]
+        step = torch.clamp(diff.abs(), max=0.005)
+        ev = self.edges[key] + torch.where(diff > 0, step, -step)
+        self.edges[key] = ev
+        h = self.inf - 3.0
+        e1, e2 = y2 - y1, (ev - y2) / h
+        w1, w2 = 2.0 * h + 1.0, h + 2.0
+        s2 = torch.where(e1 * e2 > 0, (w1 + w2) / (w1 / e1 + w2 / e2), torch.zeros_like(e1))
+        # the slope at the far end is zero (the stored edge repeats)
+        dz, dd = (e2 - s2) / h, (0.0 - e2) / h
+        out = y2 + (s2 + ((2.0 * dz - dd) + (dd - dz) / h))
+        return torch.where((y2 - out).abs() < 1e-4, y2, out)
+
+    def limit(self, dl, dr):
+        if self.lim == "vanleer":
+            t = torch.clamp(dl * dr, min=0.0) / (dl + dr)
+            return torch.nan_to_num(t, nan=0.0, posinf=math.inf, neginf=-math.inf)
+        if self.lim == "superbee":
+            cf = (dl.abs() < dr.abs()).double()
+            dl, dr = (1.0 + cf) * dl, (2.0 - cf) * dr
+        return 0.125 * (torch.sign(dl) + torch.sign(dr)) * torch.minimum(dl.abs(), dr.abs())
+
+    def b2(self):
+        return sum(c * c for c in self.c) if self.mhd else 0.0
+
+    def thermal(self, q):
+        v2 = (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / (q[0] * q[0])
+        return (self.g - 1.0) * (q[4] - 0.5 * q[0] * v2)
+
+    def gas(self):
+        return torch.clamp(self.thermal(self.q) - (self.g - 1.0) * 0.5 * self.b2(), min=0.0)
+
+    def sound(self, q, r):
+        b2 = self.b2()
+        return torch.sqrt(((self.g * (r - (self.g - 1.0) * 0.5 * b2) + 2.0 * b2) / q[0]).abs())
+
+    def flows(self, q, d):
+        """w of the five fields times the freezing speed, and that speed of each pencil."""
+        r = self.thermal(q)
+        c = self.sound(q, r)
+        p = torch.clamp(r + 0.5 * (2.0 - self.g) * self.b2(), min=0.0)
+        u = q[1 + d] / q[0]
+        speed = (u.abs() + c).amax(2 - d, keepdim=True)
+        if self.src:
+            vm = torch.clamp(self.shift(q[1 + d], d, 1) - q[1 + d], max=0.0)
+            p = p + vm * (self.src["linear"] * c + self.src["quadratic"] * vm / q[0])
+        w = [q[1 + d]]
+        for k in range(3):
+            t = u * q[1 + k]
+            if k == d:
+                t = t + p
+            w.append(t - self.c[d] * self.c[k] if self.mhd else t)
+        t = u * (q[4] + p)
+        if self.mhd:
+            t = t - self.c[d] * sum(self.c[k] * q[1 + k] for k in range(3)) / q[0]
+        return w + [t], speed
+
+    def fluid(self, d):
+        q, f = self.q, self.dt / self.dx[d]
+        w, c = self.flows(q, d)
+        half = []
+        for v in range(5):
+            t = w[v] / c
+            fr, fl = 0.5 * (q[v] + t), 0.5 * (q[v] - t)
+            self.assign(("sr", v), fr)
+            self.assign(("sl", v), fl)
+            half.append(q[v] - 0.5 * f * c * (fr - self.shift(fr, d, -1, ("sr", v)) + fl
+                                              - self.shift(fl, d, 1, ("sl", v))))
+        half[0] = torch.clamp(half[0], min=self.minmass)
+        w, c = self.flows(half, d)
+        for v in range(5):
+            t = w[v] / c
+            fr, fl = 0.5 * (half[v] + t), 0.5 * (half[v] - t)
+            r, l = ("r", v), ("l", v)
+            self.assign(r, fr)
+            self.assign(l, fl)
+            fr2 = fr + self.limit(fr - self.shift(fr, d, -1, r), self.shift(fr, d, 1, r) - fr)
+            fl2 = fl + self.limit(self.shift(fl, d, -1, l) - fl, fl - self.shift(fl, d, 1, l))
+            q[v] = q[v] - f * c * (fr2 - self.shift(fr2, d, -1, r) + fl2 - self.shift(fl2, d, 1, l))
+        q[0] = torch.clamp(q[0], min=self.minmass)
+
+    def magnet(self, x, comps):
+        s = self.shift
+        for i in comps:
+            rho, mom, b = self.q[0], self.q[1 + x], self.b[i]
+            vg = (s(mom, i, -1) + mom) / (s(rho, i, -1) + rho)
+            vg = 0.25 * (s(vg, x, -1) + s(vg, x, 1) + 2.0 * vg)
+            vf = ((vg + s(vg, x, 1)) < 0).double()
+            ff = 0.5 * self.dt / self.dx[x]
+            w = b * vg
+            w = w * (1.0 - vf) + s(w, x, 1) * vf
+            w = (b - ff * (w - s(w, x, -1))) * vg
+            up = s(w, x, 1)
+            flux = w * (1.0 - vf) + up * vf
+            dr = up - (vf * s(w, x, 2) + (1.0 - vf) * w)
+            dl = w - (vf * up + (1.0 - vf) * s(w, x, -1))
+            flux = flux + self.limit(dl, dr)
+            self.b[i] = b - 2.0 * ff * (flux - s(flux, x, -1))
+            flux = flux - s(flux, i, 1)
+            self.b[x] = self.b[x] - self.dt / self.dx[i] * s(flux, x, -1)
+        for k in (comps[1], x):
+            self.c[k] = 0.5 * (self.b[k] + s(self.b[k], k, 1))
+
+    def source(self):
+        q, a = self.q, self.src["exponent"]
+        th, es = self.src["threshold"], 0.0
+        rho = q[0] * (q[0] > th).double()
+        for d in range(self.ndims):
+            s = lambda m: self.shift(self.phi, d, m)  # noqa: B023,E731
+            ms = self.dt * rho * ((-s(2) + 8.0 * s(1) - 8.0 * s(-1) + s(-2)) / (12.0 * self.dx[d]))
+            es = es + ms * q[1 + d] / q[0]
+            q[1 + d] = q[1 + d] - ms
+        q[4] = q[4] - es
+        q[4] = q[4] - self.dt * self.strength * q[0] ** (2.0 - a) * self.gas() ** a
+
+    def iterate(self, it):
+        c = self.sound(self.q, self.thermal(self.q))
+        speeds = [float(((self.q[1 + k] / self.q[0]).abs() + c).max()) for k in range(3)]
+        k = max(range(3), key=lambda j: speeds[j])
+        self.dt = self.cfl * self.dx[k] / speeds[k]
+        if self.time + 2.0 * self.dt > self.time_max:
+            self.dt, self.time = (self.time_max - self.time) / 2.0, self.time_max
+        else:
+            self.time = self.time + 2.0 * self.dt
+        row = PERMS[(it - 1) % 6]
+        for order in (1, -1):
+            for p in row:
+                x = p if order > 0 else 4 - p
+                if self.n[x - 1] < 3:
+                    continue
+                comps = [i - 1 for i in FORWARD[x]][::order]
+                if order > 0:
+                    self.fluid(x - 1)
+                if self.mhd:
+                    self.magnet(x - 1, comps)
+                if order < 0:
+                    self.fluid(x - 1)
+            if self.src:
+                self.source()
+
+    def fields(self):
+        return [a.cpu().numpy() for a in self.q + (self.b if self.mhd else [])]
+
+
+def _noise(seed, counter):
+    """Uniform values in [-1, 1) of the counter-based generator splitmix64."""
+    z = np.uint64(seed) + np.uint64(0x9E3779B97F4A7C15) * (counter + np.uint64(1))
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    z = z ^ (z >> np.uint64(31))
+    return (z >> np.uint64(11)).astype(np.float64) * (2.0 / 9007199254740992.0) - 1.0
+
+
+def _device_state(ini, kind, params):
+    """The states that init_problem makes on the device, by its documented formulas."""
+    nx, ny, nz = ini["grid"]
+    shape, g = (nz, ny, nx), ini["gamma"]
+    mom, mag = [np.zeros(shape) for _ in range(3)], [np.zeros(shape) for _ in range(3)]
+    if kind == "orszag_tang":
+        x, y = np.arange(nx)[None, None, :] * ini["dGrid"][0], np.arange(ny)[None, :, None] * ini["dGrid"][0]
+        b0 = 1.0 / math.sqrt(4.0 * math.pi)
+        mass = np.full(shape, 25.0 / (36.0 * math.pi))
+        mom[0] = mom[0] - mass * np.sin(y)
+        mom[1] = mom[1] + mass * np.sin(x)
+        mag[0] = mag[0] - b0 * np.sin(y)
+        mag[1] = mag[1] + b0 * np.sin(2.0 * x)
+        ener = (5.0 / (12.0 * math.pi) / (g - 1.0) + 0.5 * (mom[0] ** 2 + mom[1] ** 2) / mass
+                + 0.5 * (mag[0] ** 2 + mag[1] ** 2))
+    elif kind == "sod":
+        right = np.arange(nx)[None, None, :] >= int(math.floor(nx / 2.0 + 0.5)) - 1
+        mass = np.where(right, 0.125, 1.0) + mom[0]
+        ener = np.where(right, 0.1, 1.0) / (g - 1.0) + mom[0]
+    elif kind == "sedov":
+        dx = ini["dGrid"][0]
+        c = ((np.arange(nx) + 0.5) * dx - 0.5) ** 2
+        inside = (c[:, None, None] + c[None, :, None]) + c[None, None, :] <= (params[0] * dx) ** 2
+        mass = np.ones(shape)
+        ener = np.full(shape, params[1] / (g - 1.0))
+        ener[inside] += params[2] / (inside.sum() * dx ** 3)
+    else:
+        mach, ratio, amp, seed = params
+        speed = mach * math.sqrt((g / (g - 1.0)) / (1.0 / (g - 1.0) + g * mach * mach / 2.0))
+        low = np.arange(ny)[None, :, None] >= math.ceil(ny / 2.0) - 1
+        cell = np.arange(nx * ny * nz, dtype=np.uint64).reshape(shape)
+        mass = np.where(low, 1.0 / ratio, 1.0) + mom[0]
+        mom[0] = mass * (np.where(low, -speed, speed) * (1.0 + amp * _noise(seed, np.uint64(2) * cell)))
+        mom[1] = mass * (amp * speed * _noise(seed, np.uint64(2) * cell + np.uint64(1)))
+        ener = 1.0 / (g - 1.0) + 0.5 * (mom[0] ** 2 + mom[1] ** 2) / mass
+    return {"mass": mass, "mom": mom, "ener": ener, "mag": mag}
+
+
+def exact(case, seed):
+    kind, rng = case["kind"], np.random.default_rng(seed)
+    if kind == "ensemble":
+        return None  # hundreds of simulations one after another: minutes
+    if kind == "serve":
+        out = {}
+        for i, (ini, ic, params) in enumerate(_requests(case, rng)):
+            sim, it = _Exact(ini, _device_state(ini, ic, params)), 1
+            while sim.time < sim.time_max:
+                sim.iterate(it)
+                it += 1
+            out["r%d" % i] = np.stack(sim.fields())
+        return out
+    if kind in DEVICE_STATES:
+        make, ic = DEVICE_STATES[kind]
+        ini, params = make(case, rng)
+        sim = _Exact(ini, _device_state(ini, ic, params))
+    else:
+        sim = _Exact(*HOST_STATES[kind](case, rng))
+    for it in range(1, case["iterations"] + 1):
+        sim.iterate(it)
+    return dict(zip(_fields(ini) if kind in DEVICE_STATES else FLUID + (MAGNET if sim.mhd else []),
+                    sim.fields()))
