@@ -147,7 +147,8 @@ def _mhd3d(case, rng):
     full = np.zeros((nz, ny, nx))
     ini, _ = problems.orszag_tang(4, limiter=case["limiter"], iter_max=FOREVER)
     ini["grid"] = (nx, ny, nz)
-    ini["dGrid"] = tuple(2.0 * math.pi / n for n in (nx, ny, nz))
+    # cubic cells: the time step takes the spacing of the fastest direction
+    ini["dGrid"] = (2.0 * math.pi / max(nx, ny, nz),) * 3
     mass = 1.0 + 0.2 * np.sin(x + ph[0]) * np.cos(y + z + ph[1]) + full
     vel = [0.5 * np.sin(y + ph[2]) + full, 0.5 * np.sin(z + ph[3]) + full,
            0.5 * np.sin(x + ph[4]) + full]
@@ -167,7 +168,7 @@ def _source(case, rng):
     full = np.zeros((nz, ny, nx))
     ini, _ = problems.sod(4, limiter=case["limiter"], iter_max=FOREVER)
     ini["grid"] = (nx, ny, nz)
-    ini["dGrid"] = (1.0 / nx, 1.0 / ny, 1.0 / nz)
+    ini["dGrid"] = (1.0 / max(nx, ny, nz),) * 3
     ini["bcMode"] = {"x": "circ", "y": "circ", "z": "const"}
     mass = np.exp(-0.5 * z) * (1.0 + 0.1 * np.sin(x + ph[0]) * np.sin(y + ph[1])) + full
     vel = [0.2 * np.sin(y + ph[2]) + full, 0.2 * np.cos(x + ph[0]) + full,
