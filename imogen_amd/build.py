@@ -29,6 +29,7 @@ SOURCES = ["magnet_dispatch.hip", "cfl.hip", "fluid_dispatch.cpp", "fluid_column
            "lane1d.hip", "fluid_long.hip"]
 FP32_ONLY = ("lane1d.hip",)
 VARIANT_SRC = "fluid_sweep_variant.hip"
+LEAN_VARIANT_SRC = "fluid_lean_variant.hip"
 WAVE_VARIANT_SRC = "fluid_wave_variant.hip"
 MAG_VARIANT_SRC = "magnet_sweep_variant.hip"
 
@@ -69,6 +70,7 @@ def units():
         out.append((VARIANT_SRC, "fluid_sweep_v%d_%d_%d" % (e, b, k),
                     ["-DIMH_FLUID_ESZ=%d" % e, "-DIMH_FLUID_BS=%d" % b, "-DIMH_FLUID_KMAX=%d" % k]
                     + (fp32 if e == 4 else [])))
+        out.append((LEAN_VARIANT_SRC, "fluid_lean_v%d_%d_%d" % (e, b, k), list(out[-1][2])))
     for e, b, f in wave_variants():
         # FP64 units keep contraction off: the exact ones for bit parity with the
         # restatement, the fast ones because contracted builds of this kernel gave wrong
@@ -118,7 +120,7 @@ def build(verbose=False, jobs=None, incremental=False, out=None, defines=()):
     os.makedirs(build_dir, exist_ok=True)
     us = units()
     # the long fluid variants first, so they overlap with the short units
-    us.sort(key=lambda u: 0 if u[0] in (VARIANT_SRC, MAG_VARIANT_SRC, WAVE_VARIANT_SRC) else 1)
+    us.sort(key=lambda u: 0 if u[0] in (VARIANT_SRC, LEAN_VARIANT_SRC, MAG_VARIANT_SRC, WAVE_VARIANT_SRC) else 1)
     jobs = jobs or min(len(us), max(1, (os.cpu_count() or 2)))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         results = list(ex.map(lambda u: _compile(u, verbose, incremental, defines, build_dir), us))

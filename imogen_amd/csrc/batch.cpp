@@ -49,7 +49,8 @@ struct Launch {
     int step;       // finalize: 1 or 2; source: the simulation
     int bs, kmax;   // fluid / magnet variant
     bool mhd;
-    bool general;   // fluid: the kernel form with fade boundaries / first assignments
+    bool general;   // fluid: the general kernel form, else the lean one
+    int d, px;      // fluid, lean form: sweep dimension, most pencils of a tile
     size_t smem;
     long long off;  // into the tile array
     int ntiles;
@@ -407,11 +408,12 @@ static int build_plans(imh_batch* b) {
             }
             for (int t = 0; t < 3; ++t)
                 for (int o = 0; o < 2; ++o) {
-                    // fluid groups keyed by (bs, kmax, mhd, general)
+                    // fluid groups keyed by (bs, kmax, mhd, general, and d in the lean form)
                     struct G {
                         int lane;
                         int bs, kmax;
                         bool mhd, general;
+                        int d, px;
                         double bytes;
                         std::vector<std::pair<int, BatchTile>> tl;
                     };
@@ -431,24 +433,26 @@ static int build_plans(imh_batch* b) {
                         if (c->n[X - 1] < 3) continue;
                         const bool fluid_op = (order > 0) ? (o == 0) : (o == 1);
                         if (fluid_op && c->cfg.fluid_active) {
-                            const FluidTile& ft = c->ftile[X - 1];
                             const int dX = X - 1;
-                            const bool gen = c->cfg.bc[0][dX] == IMH_BC_FADE ||
-                                             c->cfg.bc[1][dX] == IMH_BC_FADE || c->visc_type ||
-                                             c->dline_dev[dX];
+                            bool gen = c->cfg.bc[0][dX] == IMH_BC_FADE ||
+                                       c->cfg.bc[1][dX] == IMH_BC_FADE || c->visc_type ||
+                                       c->dline_dev[dX];
+                            const FluidTile& ft = fluid_tile(c, dX, gen);
                             // bs 0: the column march (one thread per pencil)
-                            const bool col = ft.column && !gen && !c->dline_dev[dX];
+                            const bool col = ft.column && !gen;
+                            if (!col && ft.PX > LEAN_PXMAX) gen = true;
                             const int gbs = col ? 0 : ft.bs, gkm = col ? 0 : ft.kmax;
+                            const int gd = (col || gen) ? 0 : dX;
                             G* g = nullptr;
                             for (G& gg : groups)
                                 if (gg.lane == lane[i] && gg.bs == gbs && gg.kmax == gkm &&
-                                    gg.mhd == c->mhd_kernel &&
-                                    gg.general == gen)
+                                    gg.mhd == c->mhd_kernel && gg.general == gen && gg.d == gd)
                                     g = &gg;
                             if (!g) {
-                                groups.push_back({lane[i], gbs, gkm, c->mhd_kernel, gen, 0.0, {}});
+                                groups.push_back({lane[i], gbs, gkm, c->mhd_kernel, gen, gd, 1, 0.0, {}});
                                 g = &groups.back();
                             }
+                            g->px = std::max(g->px, ft.PX);
                             g->bytes += double(10 + (c->mhd_kernel ? 3 : 0)) * c->ncell * es;
                             const long long per = col ? fluid_column_pencils() : ft.PX;
                             // pencil slots: pairs with a lower wormhole boundary
@@ -500,6 +504,8 @@ static int build_plans(imh_batch* b) {
                         f.kmax = g.kmax;
                         f.mhd = g.mhd;
                         f.general = g.general;
+                        f.d = g.d;
+                        f.px = g.px;
                         f.bytes = g.bytes;
                         std::vector<BatchTile> tl = sorted(g.tl);
                         add_launch(p, f, tl);
@@ -579,8 +585,11 @@ static hipError_t run_launch(imh_batch* b, const Launch& L, hipStream_t st) {
         if (L.bs == 0)
             return launch_fluid_column<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.mhd,
                                           st);
-        return launch_fluid_batch<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.bs, L.kmax,
-                                     L.mhd, L.general, st);
+        if (L.general)
+            return launch_fluid_batch<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.bs,
+                                         L.kmax, L.mhd, st);
+        return launch_fluid_lean<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.bs, L.kmax,
+                                    L.d, L.mhd, L.px, st);
     case L_MAG_ADV:
         return launch_magnet_batch<T>(0, (const MagnetArgs<T>*)b->margs, tl, L.ntiles, nb, L.kmax,
                                       L.smem, st);

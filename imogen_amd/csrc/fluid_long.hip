@@ -25,7 +25,6 @@
 // from per-pencil end values (fade_at); artificial viscosity (ArtificialViscosity.m) adds
 // a per-pencil ghost replay and a per-cell term before the predictor and the corrector.
 // A lower wormhole boundary is not taken here.
-#define IMH_FLUID_NO_LAUNCHER
 #include "fluid_sweep_impl.h"
 
 namespace imh {

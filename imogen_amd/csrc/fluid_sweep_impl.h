@@ -1,4 +1,7 @@
-// fluid_sweep_impl.h -- one fused kernel per directional fluid sweep (relaxingFluid.m).
+// fluid_sweep_impl.h -- one fused kernel per directional fluid sweep (relaxingFluid.m), in
+// its general form: fade ends, the first sweep of a simulation (first assignments of the
+// flux objects), artificial viscosity, spacing lines, and every boundary mode.  Sweeps that
+// need none of the former take fluid_lean_impl.h.
 //
 // A workgroup of BS threads owns PX whole pencils along the sweep dimension; each pencil
 // is split over TL = BS/PX threads and each thread keeps a contiguous chunk of K <= KMAX
@@ -15,6 +18,7 @@
 // Evaluation order of every expression follows the .m text, so the FP64 instantiation
 // reproduces the CPU restatement of the reference when built without FP contraction.
 #include "fluid_math.h"
+#include "fluid_tile.h"
 #include "imh_common.h"
 #include "imh_kernels.h"
 
@@ -181,65 +185,10 @@ __device__ __forceinline__ T pencil_reduce_max(T v, int xmajor, int TL, int PX, 
 
 }  // namespace
 
-// K consecutive cells as 16-byte (or one 8-byte) vector accesses; p is aligned to
-// K * sizeof(T) bytes.
-template <typename T, int K>
-__device__ __forceinline__ void chunk_load(const T* p, T (&out)[K]) {
-    constexpr int B = K * int(sizeof(T));
-    if constexpr (B % 16 == 0) {
-        constexpr int L = 16 / int(sizeof(T));
-        typedef T V __attribute__((ext_vector_type(L)));
-#pragma unroll
-        for (int j = 0; j < K / L; ++j) {
-            const V x = *gmem(reinterpret_cast<const V*>(p + j * L));
-#pragma unroll
-            for (int l = 0; l < L; ++l) out[j * L + l] = x[l];
-        }
-    } else if constexpr (B == 8 && K == 2) {
-        typedef T V __attribute__((ext_vector_type(2)));
-        const V x = *gmem(reinterpret_cast<const V*>(p));
-        out[0] = x[0];
-        out[1] = x[1];
-    } else {
-#pragma unroll
-        for (int k = 0; k < K; ++k) out[k] = gmem(p)[k];
-    }
-}
-
-template <typename T, int K>
-__device__ __forceinline__ void chunk_store(T* p, const T (&in)[K]) {
-    constexpr int B = K * int(sizeof(T));
-    if constexpr (B % 16 == 0) {
-        constexpr int L = 16 / int(sizeof(T));
-        typedef T V __attribute__((ext_vector_type(L)));
-#pragma unroll
-        for (int j = 0; j < K / L; ++j) {
-            V x;
-#pragma unroll
-            for (int l = 0; l < L; ++l) x[l] = in[j * L + l];
-            *gmem(reinterpret_cast<V*>(p + j * L)) = x;
-        }
-    } else if constexpr (B == 8 && K == 2) {
-        typedef T V __attribute__((ext_vector_type(2)));
-        V x;
-        x[0] = in[0];
-        x[1] = in[1];
-        *gmem(reinterpret_cast<V*>(p)) = x;
-    } else {
-#pragma unroll
-        for (int k = 0; k < K; ++k) gmem(p)[k] = in[k];
-    }
-}
-
 // Fields handled per exchange phase: their FR / FL live in registers across the phase's
 // barriers, so FP32 chunks of 8 cells (and FP64 of 4) take them in smaller groups.
-// IMH_FLUID_GROUP (1, 2 or 5) overrides the choice at build time.
-#ifndef IMH_FLUID_GROUP
-#define IMH_FLUID_GROUP 0
-#endif
 template <typename T, int KMAX>
 constexpr int fluid_group() {
-    if (IMH_FLUID_GROUP > 0) return IMH_FLUID_GROUP;
     return (int(sizeof(T)) * KMAX <= 16) ? 5 : (int(sizeof(T)) * KMAX <= 32 ? 2 : 1);
 }
 
@@ -263,18 +212,13 @@ constexpr int fluid_group() {
 // and the pencil ends (for the BC) in LDS, barrier, evaluate all pencil-end ghosts of
 // the group in parallel (one lane per pencil, field and shift call), barrier, update.
 //
-// GEN = false is the common case and keeps the kernel free of calls (calls cost
-// registers): no fade boundary and no first assignment of the flux objects.  GEN = true
-// handles those too, with their code out of line.
-//
-// PXM: the most pencils a tile holds (the size of the per-pencil LDS arrays; the 1-D
-// lane's tiles hold one).  GF > 0: fields per group instead of fluid_group's choice.
-template <typename T, int BS, int KMAX, bool MHD, bool GEN, int PXM = PXMAX, int GF = 0>
+template <typename T, int BS, int KMAX, bool MHD>
 __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long long tile) {
     const FluidArgs<T> a = ap;  // private copy: stores to the fields cannot alias it
     if (!a.force && !a.sim->active) return;
     using M = FMath<T>;
-    constexpr int G = GF > 0 ? GF : fluid_group<T, KMAX>();
+    constexpr int G = fluid_group<T, KMAX>();
+    constexpr int PXM = PXMAX;
     constexpr int K = KMAX;
     // chunk boundary values of the group: [field*4 + q], q = 0 first FR, 1 last FR,
     // 2 first FL, 3 last FL
@@ -287,13 +231,13 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
     __shared__ double s_trk[PXM][32];
     // artificial viscosity (general form only): first momentum value of each chunk, the
     // pencil ends of the momentum row and its upper ghost
-    __shared__ T s_mv[GEN ? BS : 1];
-    __shared__ double s_vend[GEN ? PXM : 1][6];
-    __shared__ double s_vgh[GEN ? PXM : 1];
+    __shared__ T s_mv[BS];
+    __shared__ double s_vend[PXM][6];
+    __shared__ double s_vgh[PXM];
     // Caramana-Shashkov-Whalen rows at the chunk edges (S first/last, m first/last, V at
     // k = 0, 1, K-2, K-1) and at the pencil ends (cells 0..2, N-3..N-1)
-    __shared__ T s_cw[GEN ? 8 : 1][GEN ? BS : 1];
-    __shared__ double s_cend[GEN ? PXM : 1][3][6];
+    __shared__ T s_cw[8][BS];
+    __shared__ double s_cend[PXM][3][6];
 
     const int tid = threadIdx.x;
     const int PX = a.PX, TL = a.TL;
@@ -342,7 +286,7 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
     const int mlo = mode_at(a.modes, 0, d), mhi = mode_at(a.modes, 1, d);
     const bool trk_lo = (mlo == IMH_BC_TRANS || mlo == IMH_BC_WALL);
     const bool trk_hi = (mhi == IMH_BC_TRANS || mhi == IMH_BC_WALL);
-    const bool fade = GEN && (mlo == IMH_BC_FADE || mhi == IMH_BC_FADE);
+    const bool fade = (mlo == IMH_BC_FADE || mhi == IMH_BC_FADE);
     // circular and constant boundaries need only a[0] and a[N-1] of a row: the first value
     // of the first chunk and the last value of the last chunk
     const bool simple_bc = (mlo == IMH_BC_CIRC || mlo == IMH_BC_CONST) &&
@@ -402,7 +346,6 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
     // First assignment of a flux object (InitializedArray.m:43-47): record its edges on
     // the faces of the other dimensions.
     auto init_faces = [&](int obj, const T (&vals)[K]) __attribute__((always_inline)) {
-        if constexpr (!GEN) return;
         if (!a.init_edges || a.ndims < 2) return;
 #pragma unroll
         for (int k = 0; k < K; ++k)
@@ -455,28 +398,15 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
                 s_gh[p][gv][j] = (v == X) ? -w : w;
                 continue;
             }
-            if (GEN && a.init_edges && kind < 2) s_trk[p][slot] = upper ? e[5] : e[0];
+            if (a.init_edges && kind < 2) s_trk[p][slot] = upper ? e[5] : e[0];
             double gval;
             if (mode == IMH_BC_CIRC) gval = upper ? e[0] : e[5];
             else if (mode == IMH_BC_CONST || mode == IMH_BC_FADE) gval = upper ? e[5] : e[0];
             else {
                 const int ft = which ? FT_FLUXL : FT_FLUXR;
                 const int zero_ghost = upper ? (ft != FT_FLUXR) : (ft != FT_FLUXL);
-                if constexpr (GEN) {
-                    gval = fluid_ghost(mode, upper, v == X, zero_ghost, a.active_lin, f, e[0],
-                                       e[1], e[2], e[3], e[4], e[5], N, &s_trk[p][slot]);
-                } else {
-                    GhostSpec sp;
-                    sp.mode = mode;
-                    sp.upper = upper;
-                    sp.flip_sign = (v == X);
-                    sp.zero_ghost = zero_ghost;
-                    sp.active_linear = a.active_lin;
-                    sp.bc_infinity = f;
-                    const Ends en = {e[0], e[1], e[2], e[3], e[4], e[5]};
-                    double g1;
-                    ghost_values(sp, en, N, 1, &s_trk[p][slot], gval, g1);
-                }
+                gval = fluid_ghost(mode, upper, v == X, zero_ghost, a.active_lin, f, e[0],
+                                   e[1], e[2], e[3], e[4], e[5], N, &s_trk[p][slot]);
             }
             s_gh[p][gv][j] = gval;
         }
@@ -506,7 +436,6 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
 
     // fade_shift.m blend of a shifted value at cell i (lower: shift(X,-1))
     auto fade_fix = [&](bool lower, int which, int gv, int i, T r) __attribute__((always_inline)) -> T {
-        if constexpr (!GEN) return r;
         const int mode = lower ? mlo : mhi;
         if (mode == IMH_BC_FADE && (i < f || i >= N - f) && i < N) {
             const double* e = s_ends[which][gv][px];
@@ -611,9 +540,6 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
     // of each side in the .m text's order and leaves the five values the cells read there
     // (massB/C, sndB/C, v0, v1 / v2, v3), staged in the exchange rows s_x (unused here).
     auto csw = [&](const T (&Q)[5][K], int obj) __attribute__((always_inline)) {
-      // the body exists in the general form only: left in the common form it changes that
-      // form's register allocation although it is never called there
-      if constexpr (GEN) {
         const T G = T(g);
         T Sr[K], Mr[K], Vr[K];
 #pragma unroll
@@ -735,58 +661,55 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
         }
         // the group loop that follows writes the exchange rows
         if (trk_any) __syncthreads();
-      }
     };
     auto viscosity = [&](const T (&Q)[5][K], int obj, bool first) __attribute__((always_inline)) {
-        if constexpr (GEN) {
-            if (a.visc_type == 0) return;
-            if (a.visc_type == 2) {
-                csw(Q, obj);
-                return;
-            }
-            T mX[K];
+        if (a.visc_type == 0) return;
+        if (a.visc_type == 2) {
+            csw(Q, obj);
+            return;
+        }
+        T mX[K];
 #pragma unroll
-            for (int k = 0; k < K; ++k) mX[k] = sel3(d, Q[1][k], Q[2][k], Q[3][k]);
-            s_mv[tid] = mX[0];
-            if (pen_ok) {
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    const int gi = i0 + k;
-                    if (gi < 3 && gi < N) s_vend[px][gi] = double(mX[k]);
-                    if (gi >= N - 3 && gi < N) s_vend[px][3 + gi - (N - 3)] = double(mX[k]);
-                }
-            }
-            __syncthreads();
-            if (tid < PX && slot_face(tid) >= 0) {
-                const double* e = s_vend[tid];
-                const bool trk = (mhi == IMH_BC_TRANS || mhi == IMH_BC_WALL);
-                double* tp = trk ? a.edges + a.eoff[((obj + X) * 2 + 1) * 3 + d] + slot_face(tid) : nullptr;
-                double tv = trk ? (first ? e[5] : *tp) : 0.0;
-                GhostSpec sp;
-                sp.mode = mhi;
-                sp.upper = 1;
-                sp.flip_sign = 1;  // the shifted array is the momentum component X
-                sp.zero_ghost = 0;
-                sp.active_linear = a.active_lin;
-                sp.bc_infinity = f;
-                const Ends en = {e[0], e[1], e[2], e[3], e[4], e[5]};
-                double g0, g1;
-                ghost_values(sp, en, N, 1, &tv, g0, g1);
-                if (trk) *tp = tv;
-                s_vgh[tid] = g0;
-            }
-            __syncthreads();
-            const T nb = s_mv[tr_];
-            const T gh = T(s_vgh[px]);
+        for (int k = 0; k < K; ++k) mX[k] = sel3(d, Q[1][k], Q[2][k], Q[3][k]);
+        s_mv[tid] = mX[0];
+        if (pen_ok) {
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                T sh = upper_of(mX, k, nb, gh);
-                if (mhi == IMH_BC_FADE && i0 + k < N)  // fade_shift.m: both ends blended,
-                                                       // v1 = a[1], vN = a[N-1]
-                    sh = fade_blend(sh, i0 + k, N, T(s_vend[px][1]), T(s_vend[px][5]), a.fade, f);
-                const T vm = fmin(sh - mX[k], T(0));  // MATLAB min(.., 0) skips NaN
-                P[k] = P[k] + vm * (T(a.visc_lin) * CS[k] + T(a.visc_quad) * vm / Q[0][k]);
+                const int gi = i0 + k;
+                if (gi < 3 && gi < N) s_vend[px][gi] = double(mX[k]);
+                if (gi >= N - 3 && gi < N) s_vend[px][3 + gi - (N - 3)] = double(mX[k]);
             }
+        }
+        __syncthreads();
+        if (tid < PX && slot_face(tid) >= 0) {
+            const double* e = s_vend[tid];
+            const bool trk = (mhi == IMH_BC_TRANS || mhi == IMH_BC_WALL);
+            double* tp = trk ? a.edges + a.eoff[((obj + X) * 2 + 1) * 3 + d] + slot_face(tid) : nullptr;
+            double tv = trk ? (first ? e[5] : *tp) : 0.0;
+            GhostSpec sp;
+            sp.mode = mhi;
+            sp.upper = 1;
+            sp.flip_sign = 1;  // the shifted array is the momentum component X
+            sp.zero_ghost = 0;
+            sp.active_linear = a.active_lin;
+            sp.bc_infinity = f;
+            const Ends en = {e[0], e[1], e[2], e[3], e[4], e[5]};
+            double g0, g1;
+            ghost_values(sp, en, N, 1, &tv, g0, g1);
+            if (trk) *tp = tv;
+            s_vgh[tid] = g0;
+        }
+        __syncthreads();
+        const T nb = s_mv[tr_];
+        const T gh = T(s_vgh[px]);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            T sh = upper_of(mX, k, nb, gh);
+            if (mhi == IMH_BC_FADE && i0 + k < N)  // fade_shift.m: both ends blended,
+                                                   // v1 = a[1], vN = a[N-1]
+                sh = fade_blend(sh, i0 + k, N, T(s_vend[px][1]), T(s_vend[px][5]), a.fade, f);
+            const T vm = fmin(sh - mX[k], T(0));  // MATLAB min(.., 0) skips NaN
+            P[k] = P[k] + vm * (T(a.visc_lin) * CS[k] + T(a.visc_quad) * vm / Q[0][k]);
         }
     };
 
@@ -830,10 +753,10 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
                     sL = fade_fix(false, 1, gg, i0 + k, sL);
                 }
                 // 0.5*fluxFactor .* tempFreeze; fluxFactor = dTime ./ DGRID{X} per cell
-                // on a non-uniform grid (general form only)
+                // on a non-uniform grid
                 T hk = hfC;
-                if constexpr (GEN)
-                    if (a.dxl) hk = T(0.5 * (dt / a.dxl[i0 + k < N ? i0 + k : N - 1])) * C;
+                if (a.dxl)
+                    hk = T(0.5 * (dt / a.dxl[i0 + k < N ? i0 + k : N - 1])) * C;
                 qh[v][k] = q[v][k] - hk * (FR[gg][k] - sR + FL[gg][k] - sL);
             }
         });
@@ -841,27 +764,25 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
     // First assignment of the StorageArrays (InitializedArray.m:43-47): their edges, read
     // only by the viscosity's shifts, come from this half step (the mass store's from the
     // array before its MINMASS floor, which is its second assignment).
-    if constexpr (GEN) {
-        if (a.init_edges) {
-            auto init_store = [&](auto VC) __attribute__((always_inline)) {
-                constexpr int v = decltype(VC)::value;
-                init_faces(OBJ_FSTORE + v, qh[v]);
+    if (a.init_edges) {
+        auto init_store = [&](auto VC) __attribute__((always_inline)) {
+            constexpr int v = decltype(VC)::value;
+            init_faces(OBJ_FSTORE + v, qh[v]);
 #pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    const int gi = i0 + k;
-                    if (!valid(k)) continue;
-                    if (gi == 0 && trk_lo)
-                        a.edges[a.eoff[((OBJ_FSTORE + v) * 2 + 0) * 3 + d] + pen] = double(qh[v][k]);
-                    if (gi == N - 1 && trk_hi)
-                        a.edges[a.eoff[((OBJ_FSTORE + v) * 2 + 1) * 3 + d] + pen] = double(qh[v][k]);
-                }
-            };
-            init_store(FieldIdx<0>{});
-            init_store(FieldIdx<1>{});
-            init_store(FieldIdx<2>{});
-            init_store(FieldIdx<3>{});
-            init_store(FieldIdx<4>{});
-        }
+            for (int k = 0; k < K; ++k) {
+                const int gi = i0 + k;
+                if (!valid(k)) continue;
+                if (gi == 0 && trk_lo)
+                    a.edges[a.eoff[((OBJ_FSTORE + v) * 2 + 0) * 3 + d] + pen] = double(qh[v][k]);
+                if (gi == N - 1 && trk_hi)
+                    a.edges[a.eoff[((OBJ_FSTORE + v) * 2 + 1) * 3 + d] + pen] = double(qh[v][k]);
+            }
+        };
+        init_store(FieldIdx<0>{});
+        init_store(FieldIdx<1>{});
+        init_store(FieldIdx<2>{});
+        init_store(FieldIdx<3>{});
+        init_store(FieldIdx<4>{});
     }
     // mass.store.array = max(mass.store.array, MINMASS)
 #pragma unroll
@@ -936,19 +857,13 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
             put_ends(0, gg, FR[gg]);
             put_ends(1, gg, FL[gg]);
         });
-        // U^n of the group's fields.  One group of all five fields (the common form with
-        // few cells per thread): the registers loaded at the start, kept live (measured:
-        // the re-read, 16-byte row segments in y sweeps and past the XCD's L2 by now,
-        // cost more than the spills of keeping them: 2-D sweep 202 -> 194 us).  Else
-        // re-read, all loads issued before the exchange: the addresses are clamped into
-        // the pencil and the pencil range, so the loads need no guard (only the stores do)
+        // U^n of the group's fields, read again: all loads issued before the exchange, the
+        // addresses clamped into the pencil and the pencil range, so they need no guard
+        // (only the stores do)
         T un_g[G][K];
         for_group(V0C, [&](auto VC, int gv) __attribute__((always_inline)) {
             constexpr int v = decltype(VC)::value;
-            if constexpr (G == 5 && !GEN) {
-#pragma unroll
-                for (int k = 0; k < K; ++k) un_g[v - V0][k] = q[v][k];
-            } else if (vec) {
+            if (vec) {
                 chunk_load<T, K>(a.q[v] + vbase, un_g[v - V0]);
             } else {
 #pragma unroll
@@ -973,8 +888,8 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
                     sL = fade_fix(false, 1, gg, i0 + k, sL);
                 }
                 T fk = ffC;
-                if constexpr (GEN)
-                    if (a.dxl) fk = T(dt / a.dxl[i0 + k < N ? i0 + k : N - 1]) * C2;
+                if (a.dxl)
+                    fk = T(dt / a.dxl[i0 + k < N ? i0 + k : N - 1]) * C2;
                 dq[k] = fk * (FR[gg][k] - sR + FL[gg][k] - sL);
             }
             T un[K];
@@ -1012,7 +927,7 @@ __device__ __forceinline__ void fluid_sweep_body(const FluidArgs<T>& ap, long lo
 // tile list (largest tiles first), so hundreds of uneven simulations share one launch.
 // With tiles == nullptr it is the sweep of the single simulation args[0], one block per
 // tile, with an XCD-aware block-to-tile map (neighbouring pencils share an L2).
-template <typename T, int BS, int KMAX, bool MHD, bool GEN>
+template <typename T, int BS, int KMAX, bool MHD>
 __global__ void __launch_bounds__(BS) IMH_FLUID_OCCUPANCY fluid_sweep_batch_kernel(const FluidArgs<T>* args,
                                                                const BatchTile* tiles,
                                                                int ntiles) {
@@ -1028,38 +943,9 @@ __global__ void __launch_bounds__(BS) IMH_FLUID_OCCUPANCY fluid_sweep_batch_kern
             if (r > 0 || (int)blockIdx.x >= ntiles) break;
             tile = args[0].xcd_remap ? xcd_tile(blockIdx.x, ntiles) : (long long)blockIdx.x;
         }
-        fluid_sweep_body<T, BS, KMAX, MHD, GEN>(args[arg], tile);
+        fluid_sweep_body<T, BS, KMAX, MHD>(args[arg], tile);
         __syncthreads();
     }
 }
-
-// ------------------------------------------------------------------------------------
-// Launcher of this translation unit's variant.  fluid_sweep_variant.hip is compiled once
-// per entry of IMH_FLUID_VARIANTS (imh_kernels.h) with IMH_FLUID_ESZ / IMH_FLUID_BS /
-// IMH_FLUID_KMAX defined, so the variants build in parallel; launch_fluid_batch
-// (fluid_dispatch.cpp) picks one per sweep dimension.
-// ------------------------------------------------------------------------------------
-#ifndef IMH_FLUID_NO_LAUNCHER
-#if IMH_FLUID_ESZ == 8
-using FluidT = double;
-#else
-using FluidT = float;
-#endif
-
-hipError_t IMH_FLUID_LAUNCHER(IMH_FLUID_ESZ, IMH_FLUID_BS, IMH_FLUID_KMAX)(
-    const void* args, const BatchTile* tiles, int ntiles, int nblocks, bool mhd, bool general,
-    hipStream_t st) {
-    const FluidArgs<FluidT>* a = (const FluidArgs<FluidT>*)args;
-#define IMH_FL(M, G)                                                                          \
-    if (mhd == M && general == G) {                                                           \
-        hipLaunchKernelGGL((fluid_sweep_batch_kernel<FluidT, IMH_FLUID_BS, IMH_FLUID_KMAX, M, G>), \
-                           dim3(nblocks), dim3(IMH_FLUID_BS), 0, st, a, tiles, ntiles);          \
-        return hipGetLastError();                                                             \
-    }
-    IMH_FL(false, false) IMH_FL(true, false) IMH_FL(false, true) IMH_FL(true, true)
-#undef IMH_FL
-    return hipErrorInvalidValue;
-}
-#endif
 
 }  // namespace imh

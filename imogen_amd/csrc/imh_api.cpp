@@ -125,9 +125,8 @@ static int next_pow2(int v) {
     return p;
 }
 
-// Tile of the fused fluid sweep for pencils of length N (fluid_sweep_impl.h).  Compiled
-// variants: FP64 (bs, kmax) in {(256,1), (256,2), (512,2), (512,4)}; FP32 in {(256,2),
-// (256,4), (512,4), (512,8)}.  Pencils along x are contiguous (threads of a pencil are
+// Tile of the general fluid sweep (fluid_sweep_impl.h) for pencils of length N, and any
+// tile pinned by the caller.  Pencils along x are contiguous (threads of a pencil are
 // adjacent lanes); along y/z several adjacent pencils share a block so that each row
 // access is a contiguous run.
 bool fluid_variant_exists(int esz, int bs, int kmax) { return fluid_variant_compiled(esz, bs, kmax); }
@@ -183,6 +182,55 @@ FluidTile choose_fluid_tile(int N, int d, int esz, const TileOverride* ov) {
     t.K = (N + t.TL - 1) / t.TL;
     if (t.K < 1) t.K = 1;
     return t;
+}
+
+// Tile of the lean fluid sweep (fluid_lean_impl.h) along d.  Where a sweep has fewer tiles
+// than the device has room for, its time is one tile's latency: few cells per thread.
+// With many tiles it is the work per cell: more cells per thread (fewer exchanges per
+// cell) while registers and LDS still leave three (FP64) or four (FP32) waves per SIMD,
+// which MHD sweeps with four FP64 cells per thread do not.  y / z pencils past 512 cells
+// take wider blocks, for rows of four adjacent pencils.  Measured (us per sweep, cells per
+// thread 1 / 2 / 4, 256-thread blocks): FP64 hydro 64x64: 7.7 / 9.7 / -, 48^3: 15.0 /
+// 16.3 / 22.1, 64^3: 22.7 / 19.2 / 24.6, 96^3: 65.9 / 47.9 / 50.4, 180^3: 437 / 290 / 256;
+// FP64 MHD 64^3: 18.0 / 16.3 / 22.9, 128^3: 92 / 66 / 91; FP32 hydro (2 / 4) 64^3:
+// 14.4 / 15.9, 96^3: 35.0 / 31.1, 180^3: 186 / 131; FP32 MHD 128^3: 43.3 / 46.1.  Blocks of
+// 256 / 512 / 1024 threads on y pencils: FP64 1024^2: 84.6 / 46.0 / -, FP32 1024^2: 50.8 /
+// 32.9 / 27.6, FP64 512^2: 22.3 / 20.0 / -.
+FluidTile choose_lean_tile(int N, int d, int esz, long long ncell, bool mhd) {
+    const bool x = d == 0;
+    TileOverride ov = {1, 256, 1, 1};
+    if (esz == 8) {
+        const bool many = !mhd && ncell > (1 << 20);
+        if (N <= 256) {
+            ov.kmax = ncell <= (1 << 17) ? 1 : (many ? 4 : 2);
+        } else if (N <= 512) {
+            ov.bs = (x || many) ? 256 : 512;
+            ov.kmax = many ? 4 : 2;
+        } else if (N <= 1024) {
+            // a few pencils: the shortest chunks that hold one
+            if (ncell < 64LL * N) ov.bs = 512, ov.kmax = 2;
+            else if (x || (mhd && N <= 768)) ov.kmax = 4;
+            else ov.bs = 512, ov.kmax = 8;
+        } else {
+            ov.bs = 512;
+            ov.kmax = N <= 2048 ? 4 : 8;
+        }
+    } else {
+        const bool many = ncell > (mhd ? (1 << 22) : (1 << 19));
+        if (N <= 256) {
+            ov.kmax = many ? 4 : 2;
+        } else if (N <= 512) {
+            ov.bs = x ? 256 : 512;
+            ov.kmax = (x && !many) ? 2 : 4;
+        } else {
+            ov.bs = x ? (N <= 1024 ? 256 : (N <= 2048 ? 512 : 1024)) : 1024;
+            ov.kmax = 4;
+        }
+    }
+    int tl = next_pow2((N + ov.kmax - 1) / ov.kmax);
+    if (tl < ov.bs / LEAN_PXMAX) tl = ov.bs / LEAN_PXMAX;
+    ov.px = ov.bs / (tl < ov.bs ? tl : ov.bs);
+    return choose_fluid_tile(N, d, esz, &ov);
 }
 
 // The column march applies along y / z when both boundaries are circular or constant.
@@ -489,18 +537,19 @@ static int ctx_configure(imh_ctx* c) {
     c->host_par.unconditional = 0;
     CHK(hipMemcpy(c->par, &c->host_par, sizeof(SimParams), hipMemcpyHostToDevice), "par upload");
     for (int d = 0; d < 3; ++d) {
-        c->ftile[d] = choose_fluid_tile(c->n[d], d, (int)es, nullptr);
+        c->gtile[d] = choose_fluid_tile(c->n[d], d, (int)es, nullptr);
+        c->ftile[d] = choose_lean_tile(c->n[d], d, (int)es, c->ncell, cfg->magnet_active != 0);
         // the column march has one thread per pencil: it pays where a sweep has many
         // pencils (3-D grids); the autotuner can switch it on for a dimension
         c->ftile[d].column = column_possible(cfg, d) && c->nface[d] >= (1 << 16);
         c->mtile[d] = choose_mag_tile(c->n[d]);
         c->long_dim[d] = false;
-        if (c->n[d] >= 3 && c->ftile[d].K > c->ftile[d].kmax) {
+        if (c->n[d] >= 3 && c->gtile[d].K > c->gtile[d].kmax) {
             // longer than a workgroup holds: the multi-launch sweep (fluid_long.hip)
             if (cfg->bc[0][d] == IMH_BC_WORMHOLE)
                 return fail(IMH_ENOTSUP, "pencils of %d cells along dim %d with a wormhole "
                             "boundary (the sweep of pencils longer than %d cells does not pair "
-                            "pencils)", cfg->grid[d], d + 1, c->ftile[d].kmax * c->ftile[d].bs);
+                            "pencils)", cfg->grid[d], d + 1, c->gtile[d].kmax * c->gtile[d].bs);
             if (cfg->magnet_active && c->n[d] > MAG_PENCIL_MAX)
                 return fail(IMH_ENOTSUP, "magnet pencils of %d cells along dim %d (at most %d)",
                             cfg->grid[d], d + 1, MAG_PENCIL_MAX);
@@ -511,14 +560,14 @@ static int ctx_configure(imh_ctx* c) {
         // a lower wormhole boundary pairs pencils inside a tile: long pencils take two
         // pencils of 256 threads per 512-thread block (more cells per thread)
         if (c->n[d] >= 3 && d < c->ndims && cfg->bc[0][d] == IMH_BC_WORMHOLE &&
-            (c->ftile[d].PX & 1)) {
+            (c->gtile[d].PX & 1)) {
             bool ok = false;
             for (int k = (c->n[d] + 255) / 256; k <= 64 && !ok; ++k) {
                 if (!fluid_variant_exists((int)es, 512, k)) continue;
                 const TileOverride ov = {1, 512, k, 2};
                 const FluidTile t = choose_fluid_tile(c->n[d], d, (int)es, &ov);
                 if (t.K <= t.kmax) {
-                    c->ftile[d] = t;
+                    c->gtile[d] = t;
                     ok = true;
                 }
             }
@@ -526,6 +575,10 @@ static int ctx_configure(imh_ctx* c) {
                 return fail(IMH_ENOTSUP, "wormhole BC along dim %d: pencils of %d cells need "
                             "a sweep tile of their own, and a wormhole pairs two pencils per "
                             "tile", d + 1, cfg->grid[d]);
+        }
+        if (d < c->ndims && cfg->bc[0][d] == IMH_BC_WORMHOLE) {
+            c->ftile[d] = c->gtile[d];
+            c->ftile[d].column = 0;
         }
     }
     c->host_iteration = 1;
@@ -828,6 +881,13 @@ FluidArgs<T> make_fluid_args(const imh_ctx* c, int d, int force) {
     for (int k = 0; k < 3; ++k) a.bc[k] = (const T*)c->f[IMH_F_CMAGX + k];
     a.edges = c->edges;
     a.eoff = c->eoff_dev;
+    for (int s = 0; s < 2; ++s) {
+        // the flux objects' stores are laid out one object after another (edges_layout)
+        const int m = c->cfg.bc[s][d];
+        if (m != IMH_BC_TRANS && m != IMH_BC_WALL) continue;
+        a.eo[s] = c->eoff[0][s][d];
+        a.eo_step = c->eoff[1][s][d] - c->eoff[0][s][d];
+    }
     a.sim = c->sim;
     a.n0 = c->n[0];
     a.n1 = c->n[1];
@@ -843,11 +903,6 @@ FluidArgs<T> make_fluid_args(const imh_ctx* c, int d, int force) {
     a.dx = c->cfg.dgrid[d];
     a.dxl = c->dline_dev[d];
     a.init_edges = c->fluid_init ? 0 : 1;
-    const FluidTile& t = c->ftile[d];
-    a.PX = t.PX;
-    a.TL = t.TL;
-    a.K = t.K;
-    a.xmajor = t.xmajor;
     a.worm = c->cfg.bc[0][d] == IMH_BC_WORMHOLE;
     a.npencil = a.worm ? worm_slots(c->n, d) : c->nface[d];
     a.bc_inf = c->cfg.bc_infinity;
@@ -857,6 +912,11 @@ FluidArgs<T> make_fluid_args(const imh_ctx* c, int d, int force) {
     a.visc_type = c->visc_type;
     a.visc_lin = c->visc_lin;
     a.visc_quad = c->visc_quad;
+    const FluidTile& t = fluid_tile(c, d, fluid_needs_general(a));
+    a.PX = t.PX;
+    a.TL = t.TL;
+    a.K = t.K;
+    a.xmajor = t.xmajor;
     return a;
 }
 template FluidArgs<double> make_fluid_args<double>(const imh_ctx*, int, int);
@@ -865,7 +925,8 @@ template FluidArgs<float> make_fluid_args<float>(const imh_ctx*, int, int);
 template <typename T>
 static int fluid_sweep_t(imh_ctx* c, int d, int force) {
     FluidArgs<T> a = make_fluid_args<T>(c, d, force);
-    const FluidTile& t = c->ftile[d];
+    const bool general = fluid_needs_general(a);
+    const FluidTile& t = fluid_tile(c, d, general);
     const void* da = imh_stage_args(c, &a, sizeof(a));
     if (!da) return IMH_EHIP;
     ProfScope ps(c, IMH_K_FLUID, double(10 + (c->mhd_kernel ? 3 : 0)) * c->ncell * sizeof(T));
@@ -880,7 +941,7 @@ static int fluid_sweep_t(imh_ctx* c, int d, int force) {
     // general form until it is.
     if (long_sweep(c, d)) {
         e = launch_fluid_long<T>(a, c->long_scratch, c->ncell, c->mhd_kernel, c->st);
-    } else if (c->sweep_kind != IMH_SWEEP_GENERAL && !fluid_needs_general(a) && !c->mhd_kernel && !a.dxl &&
+    } else if (c->sweep_kind != IMH_SWEEP_GENERAL && !general && !c->mhd_kernel &&
         wave_bc_ok(a.modes, d) && wave_tile(c->n[d], d, (int)sizeof(T), c->max_lds, &wbs, &wpx, &wtl, &wlds) &&
         (c->sweep_kind != IMH_SWEEP_AUTO_FAST || (a.npencil + wpx - 1) / wpx >= 4LL * c->num_cu)) {
         // the wave-spread sweep: its own tile in the argument block
@@ -893,13 +954,17 @@ static int fluid_sweep_t(imh_ctx* c, int d, int force) {
         const int nt = int((a.npencil + wpx - 1) / wpx);
         e = launch_fluid_wave((const FluidArgs<T>*)dw, nullptr, nt, nt, wbs,
                               c->sweep_kind != IMH_SWEEP_WAVE, d, c->mhd_kernel, wlds, c->st);
-    } else if (t.column && !fluid_needs_general(a) && !a.dxl) {
+    } else if (t.column && !general) {
         const int nt = int((a.npencil + fluid_column_pencils() - 1) / fluid_column_pencils());
         e = launch_fluid_column((const FluidArgs<T>*)da, nullptr, nt, nt, c->mhd_kernel, c->st);
+    } else if (!general && t.PX <= LEAN_PXMAX) {
+        const int nt = int((a.npencil + t.PX - 1) / t.PX);
+        e = launch_fluid_lean((const FluidArgs<T>*)da, nullptr, nt, nt, t.bs, t.kmax, d,
+                              c->mhd_kernel, t.PX, c->st);
     } else {
         const int nt = int((a.npencil + t.PX - 1) / t.PX);
         e = launch_fluid_batch((const FluidArgs<T>*)da, nullptr, nt, nt, t.bs, t.kmax,
-                               c->mhd_kernel, fluid_needs_general(a), c->st);
+                               c->mhd_kernel, c->st);
     }
     if (e != hipSuccess) return hip_fail(e, "fluid sweep launch");
     c->fluid_init = true;
@@ -1821,7 +1886,7 @@ int imh_set_fluid_tile(imh_ctx* c, int X, int bs, int kmax, int px) {
         (c->cfg.bc[0][X - 1] == IMH_BC_WORMHOLE && (t.PX & 1)))
         return fail(IMH_EINVAL, "tile (bs=%d kmax=%d px=%d) does not fit pencils of %d cells",
                     bs, kmax, px, c->n[X - 1]);
-    c->ftile[X - 1] = t;
+    c->ftile[X - 1] = c->gtile[X - 1] = t;
     for (int i = 0; i < 6; ++i) {
         if (c->graph[i]) hipGraphExecDestroy(c->graph[i]);
         c->graph[i] = nullptr;

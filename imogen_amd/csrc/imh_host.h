@@ -47,6 +47,7 @@ int hip_fail(hipError_t e, const char* what);
 int validate_config(const imh_config* c);
 void sweep_order(int iteration, int order, int perms_order, int dirs[3], int mi[3][2]);
 FluidTile choose_fluid_tile(int N, int d, int esz, const TileOverride* ov);
+FluidTile choose_lean_tile(int N, int d, int esz, long long ncell, bool mhd);
 bool fluid_variant_exists(int esz, int bs, int kmax);
 MagTile choose_mag_tile(int N);
 int column_possible(const imh_config* cfg, int d);
@@ -94,7 +95,8 @@ struct imh_ctx {
     double fade[imh::MAX_FADE] = {};
     double* fade_dev = nullptr;
     int host_iteration = 1;
-    imh::FluidTile ftile[3];
+    imh::FluidTile ftile[3];        // lean sweep (or the column march)
+    imh::FluidTile gtile[3];        // general sweep
     imh::MagTile mtile[3];
     hipGraphExec_t graph[6] = {};
     // Kernel argument blocks live in device memory (the kernels take a pointer, so one
@@ -127,6 +129,10 @@ struct imh_ctx {
 inline bool long_sweep(const imh_ctx* c, int d) {
     return c->long_dim[d] ||
            (c->visc_type == 2 && (c->cfg.bc[0][d] == IMH_BC_FADE || c->cfg.bc[1][d] == IMH_BC_FADE));
+}
+// Tile of the fluid sweep along d.
+inline const imh::FluidTile& fluid_tile(const imh_ctx* c, int d, bool general) {
+    return general ? c->gtile[d] : c->ftile[d];
 }
 
 

@@ -29,6 +29,8 @@ struct FluidArgs {
     const T* bc[3];          // cell-centred B (MagnetArray.cellMag)
     double* edges;           // edge-tracker storage
     const long long* eoff;   // [NOBJ][2][3] offsets into edges
+    // edges of flux object o (OBJ_SFR .. OBJ_FL + 4) on side s of dim d: eo[s] + o * eo_step
+    long long eo[2], eo_step;
     const SimDev* sim;       // device time state (dt, active)
     int n0, n1, n2;
     int d;                   // sweep dimension 0..2
@@ -101,12 +103,17 @@ __device__ __forceinline__ int xcd_round_tile(int r, int ntiles) {
     return t < hi ? t : -1;
 }
 
-// general: the launch may include a fade boundary or the first sweep of a simulation
-// (the kernel form that handles them out of line); otherwise the lean form.
+// The general form of the sweep (fluid_sweep_impl.h).
 template <typename T>
 hipError_t launch_fluid_batch(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
-                              int nblocks, int bs, int kmax, bool mhd, bool general,
-                              hipStream_t st);
+                              int nblocks, int bs, int kmax, bool mhd, hipStream_t st);
+constexpr int LEAN_PXMAX = 16;   // pencils per tile of the lean sweep
+// The lean form (fluid_lean_impl.h) of a sweep along d that fluid_needs_general() does not
+// send to the general form; px: the most pencils a tile of the launch holds.
+template <typename T>
+hipError_t launch_fluid_lean(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
+                             int nblocks, int bs, int kmax, int d, bool mhd, int px,
+                             hipStream_t st);
 // The column march for sweeps along y / z with circular or constant boundaries: one
 // thread per pencil, fluid_column_pencils() pencils per tile.
 template <typename T>
@@ -114,7 +121,8 @@ hipError_t launch_fluid_column(const FluidArgs<T>* args, const BatchTile* tiles,
                                int nblocks, bool mhd, hipStream_t st);
 int fluid_column_pencils();
 
-// whether a sweep of these arguments needs the general kernel form
+// whether a sweep of these arguments needs the general kernel form: the first sweep of a
+// simulation, a fade boundary, viscosity or a spacing line
 template <typename T>
 inline bool fluid_needs_general(const FluidArgs<T>& a) {
     return a.init_edges || a.visc_type || a.dxl || mode_at(a.modes, 0, a.d) == IMH_BC_FADE ||
@@ -126,14 +134,20 @@ inline bool fluid_needs_general(const FluidArgs<T>& a) {
 // register spills), FP32 with 2..8.  Pencils up to BS * KMAX cells fit one block.  Each
 // variant is its own translation unit.
 #define IMH_FLUID_VARIANTS(X) \
-    X(8, 256, 1) X(8, 256, 2) X(8, 512, 2) X(8, 512, 4) X(8, 512, 8) \
+    X(8, 256, 1) X(8, 256, 2) X(8, 256, 4) X(8, 512, 2) X(8, 512, 4) X(8, 512, 8) \
     X(4, 256, 2) X(4, 256, 4) X(4, 512, 4) X(4, 512, 8) X(4, 1024, 4)
 #define IMH_FLUID_LAUNCHER_(E, B, K) launch_fluid_v##E##_##B##_##K
 #define IMH_FLUID_LAUNCHER(E, B, K) IMH_FLUID_LAUNCHER_(E, B, K)
 #define IMH_FLUID_DECLARE(E, B, K)                                                         \
     hipError_t IMH_FLUID_LAUNCHER(E, B, K)(const void* args, const BatchTile* tiles, int ntiles, \
-                                           int nblocks, bool mhd, bool general, hipStream_t st);
+                                           int nblocks, bool mhd, hipStream_t st);
 IMH_FLUID_VARIANTS(IMH_FLUID_DECLARE)
+#define IMH_LEAN_LAUNCHER_(E, B, K) launch_fluid_lean_v##E##_##B##_##K
+#define IMH_LEAN_LAUNCHER(E, B, K) IMH_LEAN_LAUNCHER_(E, B, K)
+#define IMH_LEAN_DECLARE(E, B, K)                                                          \
+    hipError_t IMH_LEAN_LAUNCHER(E, B, K)(const void* args, const BatchTile* tiles, int ntiles, \
+                                          int nblocks, int d, bool mhd, int px, hipStream_t st);
+IMH_FLUID_VARIANTS(IMH_LEAN_DECLARE)
 bool fluid_variant_compiled(int esz, int bs, int kmax);
 
 // Wave-spread fluid sweep variants X(element size, block size, fast FP64 arithmetic)
