@@ -126,14 +126,14 @@ def trace_summary(trace_csv, bench_log):
         for k, (n, ns) in sorted(agg.items(), key=lambda t: -t[1][1]):
             print("| %s | %d | %.1f | %.1f | %.1f%% |" % (k, n, ns / 1e3, ns / n / 1e3,
                                                          100.0 * ns / tot))
-        fl = [(n, ns) for k, (n, ns) in agg.items() if k.startswith(("fluid_sweep", "fluid_wave"))]
+        fl = [(n, ns) for k, (n, ns) in agg.items() if k.startswith(("fluid_sweep", "fluid_lean"))]
         n, ns = sum(x[0] for x in fl), sum(x[1] for x in fl)
         print("\nfluid sweep: %d launches, average %.2f us per launch in the trace; "
               "bench.py (HIP events): %.2f us over %d launches\n" % (
                   n, ns / n / 1e3, ref["avg_launch_us"], ref["launches"]))
 
     def is_fluid(r, prec):
-        return (("fluid_sweep" in r["Kernel_Name"] or "fluid_wave" in r["Kernel_Name"])
+        return (("fluid_sweep" in r["Kernel_Name"] or "fluid_lean" in r["Kernel_Name"])
                 and ("<%s" % prec) in r["Kernel_Name"])
 
     if "roofline" not in out:  # a --only-plain run
@@ -201,7 +201,7 @@ def pmc_traffic(fetch_csv, write_csv, bench_log):
             if not n:
                 continue
             fl = [r for r in rows if ("fluid_sweep" in r["Kernel_Name"] or
-                                      "fluid_wave" in r["Kernel_Name"])
+                                      "fluid_lean" in r["Kernel_Name"])
                   and ("<%s" % prec) in r["Kernel_Name"]][-n:]
             kib = sum(float(r["Counter_Value"]) for r in fl)
             e = res.setdefault(out[key]["workload"] if key == "plain_roofline"
@@ -580,8 +580,7 @@ def configs_leg(args):
     return out
 
 
-# The plain FP64 path's fluid sweep: the fast FP64 wave-spread sweep where its tiles fill
-# the device, the general sweep elsewhere (include/imogen_hip_ext.h, IMH_SWEEP_AUTO_FAST).
+# The plain FP64 path's sweep kind (include/imogen_hip_ext.h, IMH_SWEEP_AUTO_FAST).
 PLAIN_SWEEP = "auto_fast"
 
 
@@ -603,7 +602,7 @@ def large_plain_roofline(args):
         res[kind] = roofline(prof, "sedov 256^3 hydro FP64, plain path")
     del st
     out = res[PLAIN_SWEEP]
-    out["sweep"] = "wave-spread sweep, fast FP64 arithmetic (%s)" % PLAIN_SWEEP
+    out["sweep"] = "lean sweep (%s)" % PLAIN_SWEEP
     out["general_sweep"] = {k: res["general"][k] for k in ("achieved", "frac", "avg_launch_us")}
     return out
 

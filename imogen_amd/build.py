@@ -30,7 +30,6 @@ SOURCES = ["magnet_dispatch.hip", "cfl.hip", "fluid_dispatch.cpp", "fluid_column
 FP32_ONLY = ("lane1d.hip",)
 VARIANT_SRC = "fluid_sweep_variant.hip"
 LEAN_VARIANT_SRC = "fluid_lean_variant.hip"
-WAVE_VARIANT_SRC = "fluid_wave_variant.hip"
 MAG_VARIANT_SRC = "magnet_sweep_variant.hip"
 
 
@@ -49,14 +48,6 @@ def magnet_variants():
     return [tuple(int(v) for v in t) for t in re.findall(r"X\((\d+), (\d+)\)", m.group(1))]
 
 
-def wave_variants():
-    """(element size, block size, fast FP64) of every wave-spread sweep variant
-    (IMH_WAVE_VARIANTS in imh_kernels.h)."""
-    text = open(os.path.join(CSRC, "imh_kernels.h")).read()
-    m = re.search(r"#define IMH_WAVE_VARIANTS\(X\)((?:[^\n]*\\\n)*[^\n]*)", text)
-    return [tuple(int(v) for v in t) for t in re.findall(r"X\((\d+), (\d+), (\d+)\)", m.group(1))]
-
-
 def units():
     """(source, object name, extra flags) of every translation unit."""
     # FP64 units keep -ffp-contract=off (the FP64 kernels reproduce the oracle's rounding);
@@ -71,13 +62,6 @@ def units():
                     ["-DIMH_FLUID_ESZ=%d" % e, "-DIMH_FLUID_BS=%d" % b, "-DIMH_FLUID_KMAX=%d" % k]
                     + (fp32 if e == 4 else [])))
         out.append((LEAN_VARIANT_SRC, "fluid_lean_v%d_%d_%d" % (e, b, k), list(out[-1][2])))
-    for e, b, f in wave_variants():
-        # FP64 units keep contraction off: the exact ones for bit parity with the
-        # restatement, the fast ones because contracted builds of this kernel gave wrong
-        # MHD sweeps along y (their arithmetic gain is the reciprocals)
-        out.append((WAVE_VARIANT_SRC, "fluid_wave_v%d_%d_%d" % (e, b, f),
-                    ["-DIMH_WAVE_ESZ=%d" % e, "-DIMH_WAVE_BS=%d" % b, "-DIMH_WAVE_FAST=%d" % f]
-                    + (fp32 if e == 4 else [])))
     for e, k in magnet_variants():
         out.append((MAG_VARIANT_SRC, "magnet_sweep_v%d_%d" % (e, k),
                     ["-DIMH_MAG_ESZ=%d" % e, "-DIMH_MAG_KMAX=%d" % k] + (fp32 if e == 4 else [])))
@@ -120,7 +104,7 @@ def build(verbose=False, jobs=None, incremental=False, out=None, defines=()):
     os.makedirs(build_dir, exist_ok=True)
     us = units()
     # the long fluid variants first, so they overlap with the short units
-    us.sort(key=lambda u: 0 if u[0] in (VARIANT_SRC, LEAN_VARIANT_SRC, MAG_VARIANT_SRC, WAVE_VARIANT_SRC) else 1)
+    us.sort(key=lambda u: 0 if u[0] in (VARIANT_SRC, LEAN_VARIANT_SRC, MAG_VARIANT_SRC) else 1)
     jobs = jobs or min(len(us), max(1, (os.cpu_count() or 2)))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         results = list(ex.map(lambda u: _compile(u, verbose, incremental, defines, build_dir), us))

@@ -189,13 +189,19 @@ FluidTile choose_fluid_tile(int N, int d, int esz, const TileOverride* ov) {
 // With many tiles it is the work per cell: more cells per thread (fewer exchanges per
 // cell) while registers and LDS still leave three (FP64) or four (FP32) waves per SIMD,
 // which MHD sweeps with four FP64 cells per thread do not.  y / z pencils past 512 cells
-// take wider blocks, for rows of four adjacent pencils.  Measured (us per sweep, cells per
-// thread 1 / 2 / 4, 256-thread blocks): FP64 hydro 64x64: 7.7 / 9.7 / -, 48^3: 15.0 /
-// 16.3 / 22.1, 64^3: 22.7 / 19.2 / 24.6, 96^3: 65.9 / 47.9 / 50.4, 180^3: 437 / 290 / 256;
-// FP64 MHD 64^3: 18.0 / 16.3 / 22.9, 128^3: 92 / 66 / 91; FP32 hydro (2 / 4) 64^3:
-// 14.4 / 15.9, 96^3: 35.0 / 31.1, 180^3: 186 / 131; FP32 MHD 128^3: 43.3 / 46.1.  Blocks of
-// 256 / 512 / 1024 threads on y pencils: FP64 1024^2: 84.6 / 46.0 / -, FP32 1024^2: 50.8 /
-// 32.9 / 27.6, FP64 512^2: 22.3 / 20.0 / -.
+// take wider blocks, for rows of four adjacent pencils (z pencils past 256 cells too:
+// their neighbouring rows lie a plane apart, and a tile's row is all that shares a cache
+// line).  Measured (us per sweep, cells per thread 1 / 2 / 4, 256-thread blocks): FP64
+// hydro 64x64: 7.7 / 9.7 / -, 48^3: 15.0 / 16.3 / 22.1, 64^3: 22.7 / 19.2 / 24.6, 96^3:
+// 65.9 / 47.9 / 50.4, 180^3: 437 / 290 / 256; FP64 MHD 64^3: 18.0 / 16.3 / 22.9, 128^3: 92
+// / 66 / 91; FP32 hydro (2 / 4) 64^3: 14.4 / 15.9, 96^3: 35.0 / 31.1, 180^3: 186 / 131;
+// FP32 MHD 128^3: 43.3 / 46.1.  FP32 MHD 256^3 in blocks of 256 / 512 (4 cells) y: 505 /
+// 426, z: 664 / 457.  Blocks of 256 / 512 / 1024 threads on y pencils: FP64 1024^2: 84.6 /
+// 46.0 / -, FP32 1024^2: 50.8 / 32.9 / 27.6, FP64 512^2: 22.3 / 20.0 / -.  3-D y and z
+// sweeps with rows of 2 / 4 / 8 pencils: FP64 512^3 y 5642 / 7465 / 6406, z 10897 / 10498
+// / 7707, 320^3 z 2533 / 2893 / 2229; FP32 512^3 y 4379 / 2935 / 3335, z 10928 / 5614 /
+// 4147.  Past 1024 cells, rows of 1 / 2 pencils in a 3-D grid (32 x 2048 x 2048): FP64
+// 12433 / 8512, FP32 8881 / 5128.
 FluidTile choose_lean_tile(int N, int d, int esz, long long ncell, bool mhd) {
     const bool x = d == 0;
     TileOverride ov = {1, 256, 1, 1};
@@ -204,8 +210,8 @@ FluidTile choose_lean_tile(int N, int d, int esz, long long ncell, bool mhd) {
         if (N <= 256) {
             ov.kmax = ncell <= (1 << 17) ? 1 : (many ? 4 : 2);
         } else if (N <= 512) {
-            ov.bs = (x || many) ? 256 : 512;
-            ov.kmax = many ? 4 : 2;
+            ov.bs = (x || (many && d == 1)) ? 256 : 512;
+            ov.kmax = many ? (d == 2 ? 8 : 4) : 2;
         } else if (N <= 1024) {
             // a few pencils: the shortest chunks that hold one
             if (ncell < 64LL * N) ov.bs = 512, ov.kmax = 2;
@@ -213,14 +219,15 @@ FluidTile choose_lean_tile(int N, int d, int esz, long long ncell, bool mhd) {
             else ov.bs = 512, ov.kmax = 8;
         } else {
             ov.bs = 512;
-            ov.kmax = N <= 2048 ? 4 : 8;
+            ov.kmax = N <= 2048 && (x || ncell < 65536LL * N) ? 4 : 8;
         }
     } else {
         const bool many = ncell > (mhd ? (1 << 22) : (1 << 19));
         if (N <= 256) {
-            ov.kmax = many ? 4 : 2;
+            ov.kmax = many && !(mhd && x) ? 4 : 2;
+            if (mhd && many && !x) ov.bs = 512;
         } else if (N <= 512) {
-            ov.bs = x ? 256 : 512;
+            ov.bs = x ? 256 : (d == 2 && many ? 1024 : 512);
             ov.kmax = (x && !many) ? 2 : 4;
         } else {
             ov.bs = x ? (N <= 1024 ? 256 : (N <= 2048 ? 512 : 1024)) : 1024;
@@ -465,15 +472,6 @@ static int ctx_alloc(imh_ctx* c) {
     const imh_config* cfg = &c->cfg;
     const size_t bytes = (size_t)c->ncell * esize(c);
     CHK(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking), "hipStreamCreate");
-    {
-        hipDeviceProp_t prop;
-        if (hipGetDeviceProperties(&prop, cfg->device) == hipSuccess && prop.multiProcessorCount > 0) {
-            c->num_cu = prop.multiProcessorCount;
-            // dynamic LDS above 64 KiB would need a per-kernel attribute: the wave-spread
-            // sweep stays within 64 KiB
-            c->max_lds = std::min<size_t>(prop.sharedMemPerBlock, 64 * 1024);
-        }
-    }
     for (int i = 0; i < IMH_NFIELDS; ++i) CHK(hipMalloc(&c->f[i], bytes), "hipMalloc(field)");
     if (cfg->magnet_active) CHK(hipMalloc(&c->scratch, bytes), "hipMalloc(scratch)");
     c->edges_cap = c->edges_len;
@@ -539,9 +537,14 @@ static int ctx_configure(imh_ctx* c) {
     for (int d = 0; d < 3; ++d) {
         c->gtile[d] = choose_fluid_tile(c->n[d], d, (int)es, nullptr);
         c->ftile[d] = choose_lean_tile(c->n[d], d, (int)es, c->ncell, cfg->magnet_active != 0);
-        // the column march has one thread per pencil: it pays where a sweep has many
-        // pencils (3-D grids); the autotuner can switch it on for a dimension
-        c->ftile[d].column = column_possible(cfg, d) && c->nface[d] >= (1 << 16);
+        // the column march (one thread per pencil, a wave's rows contiguous) where a tile of
+        // the lean sweep holds a single pencil, whose rows are single cells, and there are
+        // pencils enough to fill the device.  Shorter pencils: column / lean, us per sweep,
+        // circular FP64 256^3 1089 / 605, 384^3 4472 / 2626, 64 x 1024^2 4086 / 2973, 32 x
+        // 2048^2 9397 / 8512; FP32 695 / 303, 1538 / 1346, 2842 / 1578, 5951 / 5128.  The
+        // autotuner can switch it on for a dimension.
+        c->ftile[d].column = column_possible(cfg, d) && c->nface[d] >= (1 << 16) &&
+                             c->ftile[d].PX == 1;
         c->mtile[d] = choose_mag_tile(c->n[d]);
         c->long_dim[d] = false;
         if (c->n[d] >= 3 && c->gtile[d].K > c->gtile[d].kmax) {
@@ -640,8 +643,6 @@ int imh_ctx_recycle(imh_ctx* old, const imh_config* cfg_in, imh_ctx** out) {
     // move the device memory over; the old context keeps (and frees) everything else
     c->st = old->st;
     old->st = nullptr;
-    c->num_cu = old->num_cu;
-    c->max_lds = old->max_lds;
     for (int i = 0; i < IMH_NFIELDS; ++i) {
         c->f[i] = old->f[i];
         old->f[i] = nullptr;
@@ -931,29 +932,8 @@ static int fluid_sweep_t(imh_ctx* c, int d, int force) {
     if (!da) return IMH_EHIP;
     ProfScope ps(c, IMH_K_FLUID, double(10 + (c->mhd_kernel ? 3 : 0)) * c->ncell * sizeof(T));
     hipError_t e;
-    int wbs = 0, wpx = 0, wtl = 0;
-    size_t wlds = 0;
-    // the wave-spread sweep where it applies (with IMH_SWEEP_AUTO_FAST only where its
-    // tiles fill the device, at least 4 per CU: short sweeps keep the general form's
-    // smaller tiles)
-    // Hydro sweeps only: a run of the MHD instantiations (the only ones that spill
-    // registers to scratch) left the GPU faulted once, cause not found; MHD sweeps take the
-    // general form until it is.
     if (long_sweep(c, d)) {
         e = launch_fluid_long<T>(a, c->long_scratch, c->ncell, c->mhd_kernel, c->st);
-    } else if (c->sweep_kind != IMH_SWEEP_GENERAL && !general && !c->mhd_kernel &&
-        wave_bc_ok(a.modes, d) && wave_tile(c->n[d], d, (int)sizeof(T), c->max_lds, &wbs, &wpx, &wtl, &wlds) &&
-        (c->sweep_kind != IMH_SWEEP_AUTO_FAST || (a.npencil + wpx - 1) / wpx >= 4LL * c->num_cu)) {
-        // the wave-spread sweep: its own tile in the argument block
-        a.PX = wpx;
-        a.TL = wtl;
-        a.K = 4;
-        a.xmajor = d == 0;
-        const void* dw = imh_stage_args(c, &a, sizeof(a));
-        if (!dw) return IMH_EHIP;
-        const int nt = int((a.npencil + wpx - 1) / wpx);
-        e = launch_fluid_wave((const FluidArgs<T>*)dw, nullptr, nt, nt, wbs,
-                              c->sweep_kind != IMH_SWEEP_WAVE, d, c->mhd_kernel, wlds, c->st);
     } else if (t.column && !general) {
         const int nt = int((a.npencil + fluid_column_pencils() - 1) / fluid_column_pencils());
         e = launch_fluid_column((const FluidArgs<T>*)da, nullptr, nt, nt, c->mhd_kernel, c->st);

@@ -84,9 +84,7 @@ struct imh_ctx {
     bool obj_init[imh::NOBJ] = {};
     bool fluid_init = false;
     bool squeezed = false;   // the grid was relabelled by squeeze_grid (singleton x or y)
-    int sweep_kind = 0;             // IMH_SWEEP_GENERAL / _WAVE / _WAVE_FAST
-    int num_cu = 256;               // compute units of the device
-    size_t max_lds = 64 * 1024;     // LDS bytes per workgroup of the device
+    int sweep_kind = 0;             // IMH_SWEEP_*: as set, every kind runs the same sweep
     bool have_state = false;
     bool mhd_kernel = false;
     bool no_graphs = false;

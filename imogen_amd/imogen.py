@@ -280,9 +280,9 @@ class ImogenManager:
     SWEEP_KINDS = {"general": 0, "wave": 1, "wave_fast": 2, "auto_fast": 3}
 
     def set_fluid_kernel(self, kind):
-        """The fluid sweep kernel: 'general', 'wave' (wave-spread, the precision's own
-        arithmetic), 'wave_fast' (wave-spread, fast FP64 arithmetic) or 'auto_fast'
-        (wave_fast where its tiles fill the device, general elsewhere)."""
+        """The fluid sweep kind: 'general', 'wave', 'wave_fast' or 'auto_fast' (the last two
+        on FP64 only).  Every kind runs the same sweep, with the precision's own
+        arithmetic."""
         check(lib().imh_set_fluid_kernel(self._ctx, self.SWEEP_KINDS[kind]))
 
     def get_fluid_tile(self, X):
