@@ -18,8 +18,11 @@
 //    would be read, so the cells next to an end need no selects.
 //  * LDS: 20 rows of one value per thread, and what the PX pencils' ends need (PX known at
 //    the launch: dynamic LDS).
+//  * The argument block is read into scalar registers (uniform_load): FP64 4 cells per
+//    thread 168 vector registers with spills -> 147, 2 cells 123; FP64 256^3 664 -> 621 us per
+//    sweep, FP32 192^3 158 -> 147, a 1024-cell tube 18.0 -> 16.9.
 // Measured against the general form (us per sweep, mean of the directions): FP64 125^3 175 ->
-// 80, 256^3 1463 -> 624-664 (1.34 GB: 2.1 TB/s), 333x333 19 -> 15, FP32 192^3 372 -> 157,
+// 78, 256^3 1463 -> 621 (1.34 GB: 2.2 TB/s), 333x333 19 -> 15, FP32 192^3 372 -> 147,
 // 1024x1024 37 -> 26, FP64 MHD 96^3 61 -> 43.  Spilling registers for one more wave per SIMD
 // loses (FP64, 2 cells per thread at 4 waves: 782 -> 1130 at 256^3).
 // Every expression keeps the .m evaluation order (FP64: bit for bit the general form; FP32
@@ -239,8 +242,8 @@ __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, doubl
 // The sweep of one tile (PX pencils) of one simulation along D.  lds: lean::lds_layout.
 template <typename T, int BS, int K, bool MHD, int D>
 __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long long tile, char* lds) {
-    const FluidArgs<T> a = ap;  // private copy: stores to the fields cannot alias it
-    if (!a.force && !a.sim->active) return;
+    const FluidArgs<T> a = uniform_load(&ap);
+    if (!a.force && !uniform_load(&a.sim->active)) return;
     using M = LMath<T>;
     constexpr bool XM = D == 0;
     constexpr int X = D + 1;
@@ -298,7 +301,7 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
         return base + unsigned(i) * stride;
     };
 
-    const double dt = a.sim->dt;
+    const double dt = uniform_load(&a.sim->dt);
     const double ff = dt / a.dx;          // fluxFactor = dTime ./ DGRID{X}
     const double hf = 0.5 * ff;
     const double g = a.gamma;

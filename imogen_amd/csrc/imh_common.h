@@ -402,6 +402,26 @@ __device__ __forceinline__ IMH_GLOBAL_AS T* gmem(T* p) {
     return (IMH_GLOBAL_AS T*)p;
 }
 
+// A copy of an argument block (or a value) that is the same for all lanes and that no kernel
+// of the launch writes, through the constant address space: scalar loads into scalar
+// registers.  Read as ordinary memory in a loop that also stores, the block is loaded by
+// every lane and its pointers and sizes take vector registers, two per pointer.
+template <typename A>
+__device__ __forceinline__ A uniform_load(const A* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    static_assert(sizeof(A) % 4 == 0, "whole words");
+    struct W {
+        int w[sizeof(A) / 4];
+    } v;
+    const __attribute__((address_space(4))) int* q = (const __attribute__((address_space(4))) int*)p;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(A) / 4; ++i) v.w[i] = q[i];
+    return __builtin_bit_cast(A, v);
+#else
+    return *p;
+#endif
+}
+
 // Face index of cell (i,j,k) for dim d (same conventions).
 // Pencil slots of a sweep along d whose lower boundary is a wormhole (wormhole_shift.m):
 // the lower ghosts of the pencil at next-dimension coordinate c (next = x->y, y->z, z->x)
