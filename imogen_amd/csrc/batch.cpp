@@ -39,7 +39,8 @@ using namespace imh;
 
 namespace {
 
-enum LaunchKind { L_BEGIN, L_CFL_RESET, L_CFL, L_FINALIZE, L_FLUID, L_MAG_ADV, L_MAG_CT, L_CELLMAG, L_END,
+enum LaunchKind { L_BEGIN, L_CFL_RESET, L_CFL, L_FINALIZE, L_FLUID, L_MAG_ADV, L_MAG_CT, L_CELLMAG,
+                  L_MAG_FLOW, L_MAG_CURL, L_END,
                   L_FORK, L_JOIN, L_SOURCE, L_LANE1D };
 
 constexpr int MAX_LANES = 2;
@@ -49,8 +50,8 @@ struct Launch {
     int step;       // finalize: 1 or 2; source: the simulation
     int bs, kmax;   // fluid / magnet variant
     bool mhd;
-    bool general;   // fluid: the general kernel form, else the lean one
-    int d, px;      // fluid, lean form: sweep dimension, most pencils of a tile
+    bool general;   // fluid: the general kernel form, else the lean one; lean magnet: tracked
+    int d, px;      // lean forms: sweep dimension; fluid: most pencils of a tile
     size_t smem;
     long long off;  // into the tile array
     int ntiles;
@@ -63,8 +64,10 @@ int launch_kind_class(LaunchKind k) {
     switch (k) {
     case L_CFL: return IMH_K_CFL;
     case L_FLUID: return IMH_K_FLUID;
-    case L_MAG_ADV: return IMH_K_MAG_ADV;
-    case L_MAG_CT: return IMH_K_MAG_CT;
+    case L_MAG_ADV:
+    case L_MAG_FLOW: return IMH_K_MAG_ADV;
+    case L_MAG_CT:
+    case L_MAG_CURL: return IMH_K_MAG_CT;
     case L_CELLMAG: return IMH_K_CELLMAG;
     case L_SOURCE: return IMH_K_SOURCE;
     case L_LANE1D: return IMH_K_LANE1D;
@@ -86,6 +89,7 @@ struct imh_batch {
     SimParams** pars_dev = nullptr;
     void* fargs = nullptr;    // FluidArgs<T>[n*3]
     void* margs = nullptr;    // MagnetArgs<T>[n*9], index sim*9 + 3*dI + dX
+    void* mlargs = nullptr;   // MagnetLeanArgs<T>[n*6], index sim*6 + mlean_index(dX, I)
     void* cargs = nullptr;    // CellMagArgs<T>[n*3]
     void* cflargs = nullptr;  // CflArgs<T>[n]
     BatchTile* tiles = nullptr;
@@ -110,17 +114,19 @@ struct imh_batch {
 };
 
 // A simulation whose whole flux call runs in the 1-D lane launch (lane1d.hip): FP32
-// bulk, one pencil (N x 1 x 1, 3 <= N <= 4096), fluid and magnet both active, no source
-// terms, viscosity, fade ends or spacing lines (those take the general sweep), the time
-// step once per iteration in every simulation of the batch.
+// bulk, one pencil (N x 1 x 1, 8 <= N <= 4096), fluid and magnet both active, no source
+// terms, viscosity, fade ends or spacing lines (those take the general sweep), the lean
+// magnetic sweep's conditions, the time step once per iteration in every simulation of the
+// batch.
 static bool lane1d_ok(const imh_batch* b, const imh_ctx* c) {
     if (!b->fuse_1d || b->prec != IMH_FP32_BULK || b->any_step_mode) return false;
-    if (c->n[1] != 1 || c->n[2] != 1 || c->n[0] < 3 || c->n[0] > LANE1D_NMAX) return false;
+    if (c->n[1] != 1 || c->n[2] != 1 || c->n[0] > LANE1D_NMAX) return false;
     if (!c->cfg.fluid_active || !c->cfg.magnet_active || !c->mhd_kernel) return false;
     if (c->grav || c->rad_type || c->visc_type || c->dline_dev[0]) return false;
     for (int s = 0; s < 2; ++s)
         if (c->cfg.bc[s][0] == IMH_BC_FADE) return false;
-    return true;
+    const int I[2] = {2, 3}, J[2] = {3, 2};
+    return magnet_lean_ok(c, 0, I) && magnet_lean_ok(c, 0, J);
 }
 
 // Wait until nothing of the batch is in flight: the batch stream (graph replays join
@@ -151,6 +157,7 @@ static void batch_free(imh_batch* b) {
     hipFree(b->pars_dev);
     hipFree(b->fargs);
     hipFree(b->margs);
+    hipFree(b->mlargs);
     hipFree(b->cargs);
     hipFree(b->cflargs);
     hipFree(b->tiles);
@@ -171,14 +178,19 @@ static void batch_free(imh_batch* b) {
     delete b;
 }
 
+// The six argument blocks of the lean magnetic sweep: direction and order of the components.
+static int mlean_index(int dX, const int I[2]) { return 2 * dX + (I[0] > I[1] ? 1 : 0); }
+
 template <typename T>
 static int upload_args_t(imh_batch* b) {
     const int n = b->n;
     std::vector<FluidArgs<T>> fa(n * 3);
     std::vector<MagnetArgs<T>> ma(n * 9);
+    std::vector<MagnetLeanArgs<T>> ml(n * 6);
     std::vector<CellMagArgs<T>> ca(n * 3);
     std::vector<CflArgs<T>> cf(n);
     memset(ma.data(), 0, sizeof(MagnetArgs<T>) * ma.size());
+    memset(ml.data(), 0, sizeof(MagnetLeanArgs<T>) * ml.size());
     for (int i = 0; i < n; ++i) {
         const imh_ctx* c = b->ctx[i];
         for (int d = 0; d < 3; ++d) {
@@ -190,12 +202,22 @@ static int upload_args_t(imh_batch* b) {
             for (int dI = 0; dI < 3; ++dI)
                 for (int dX = 0; dX < 3; ++dX)
                     if (dI != dX) ma[i * 9 + 3 * dI + dX] = make_magnet_args<T>(c, dX, dI, 0);
+        if (c->cfg.magnet_active)
+            for (int dX = 0; dX < 3; ++dX)
+                for (int o = 0; o < 2; ++o) {
+                    int I[2] = {dX == 0 ? 2 : 1, dX == 2 ? 2 : 3};
+                    if (o) std::swap(I[0], I[1]);
+                    ml[i * 6 + mlean_index(dX, I)] = make_magnet_lean_args<T>(c, dX, I, 0);
+                }
         cf[i] = make_cfl_args<T>(c);
     }
     hipError_t e = hipMemcpyAsync(b->fargs, fa.data(), sizeof(FluidArgs<T>) * fa.size(),
                                   hipMemcpyHostToDevice, b->st);
     if (e == hipSuccess)
         e = hipMemcpyAsync(b->margs, ma.data(), sizeof(MagnetArgs<T>) * ma.size(),
+                           hipMemcpyHostToDevice, b->st);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(b->mlargs, ml.data(), sizeof(MagnetLeanArgs<T>) * ml.size(),
                            hipMemcpyHostToDevice, b->st);
     if (e == hipSuccess)
         e = hipMemcpyAsync(b->cargs, ca.data(), sizeof(CellMagArgs<T>) * ca.size(),
@@ -232,12 +254,11 @@ static int upload_args_t(imh_batch* b) {
                 if (N <= LANE1D_BS * (q * LANE1D_KMAX / 4)) kc = q * LANE1D_KMAX / 4;
             l.fa.K = kc;
             l.fa.xmajor = 1;
-            for (int dI = 1; dI < 3; ++dI) {
-                l.ma[dI] = ma[i * 9 + 3 * dI + 0];
-                l.ma[dI].PX = 1;
-                l.ma[dI].TL = LANE1D_BS;
+            for (int o = 0; o < 2; ++o) {
+                l.ml[o] = ml[i * 6 + o];  // X = 1: mlean_index 0 (I = [2 3]) and 1 ([3 2])
+                l.ml[o].PX = 1;
+                l.ml[o].TL = LANE1D_BS;
             }
-            for (int k = 0; k < 3; ++k) l.ca[k] = ca[i * 3 + k];
         }
         if (e == hipSuccess && la.size() > b->l1cap) {
             hipFree(b->l1args);
@@ -269,10 +290,12 @@ static int batch_setup(imh_batch* b) {
     if (e == hipSuccess) e = hipMalloc(&b->pars_dev, sizeof(SimParams*) * n);
     size_t fsz = b->prec == IMH_FP64 ? sizeof(FluidArgs<double>) : sizeof(FluidArgs<float>);
     size_t msz = b->prec == IMH_FP64 ? sizeof(MagnetArgs<double>) : sizeof(MagnetArgs<float>);
+    size_t mlsz = b->prec == IMH_FP64 ? sizeof(MagnetLeanArgs<double>) : sizeof(MagnetLeanArgs<float>);
     size_t csz = b->prec == IMH_FP64 ? sizeof(CellMagArgs<double>) : sizeof(CellMagArgs<float>);
     size_t lsz = b->prec == IMH_FP64 ? sizeof(CflArgs<double>) : sizeof(CflArgs<float>);
     if (e == hipSuccess) e = hipMalloc(&b->fargs, fsz * n * 3);
     if (e == hipSuccess) e = hipMalloc(&b->margs, msz * n * 9);
+    if (e == hipSuccess) e = hipMalloc(&b->mlargs, mlsz * n * 6);
     if (e == hipSuccess) e = hipMalloc(&b->cargs, csz * n * 3);
     if (e == hipSuccess) e = hipMalloc(&b->cflargs, lsz * n);
     if (e != hipSuccess) return hip_fail(e, "batch allocation");
@@ -419,6 +442,9 @@ static int build_plans(imh_batch* b) {
                     };
                     std::vector<G> groups;
                     std::vector<std::pair<int, BatchTile>> adv[2], ct[2];
+                    std::vector<std::pair<int, BatchTile>> flow[6], curl[6];  // lean: 2 * direction + tracked
+                    double lean_cells[6] = {};
+                    size_t lean_lds[6][2] = {};
                     std::vector<BatchTile> cm;
                     double mag_cells = 0;
                     int magkmax[2] = {1, 1};
@@ -464,6 +490,22 @@ static int build_plans(imh_batch* b) {
                                 g->tl.push_back({c->n[X - 1], {i * 3 + (X - 1), 0, tt}});
                         } else if (!fluid_op && c->cfg.magnet_active) {
                             const int dX = X - 1;
+                            if (magnet_lean_ok(c, dX, mi[t])) {
+                                const int arg = i * 6 + mlean_index(dX, mi[t]), N = c->n[dX];
+                                const int gi = 2 * dX + (magnet_lean_tracked(c) ? 1 : 0);
+                                int px, tl;
+                                mag_lean_tile(c, dX, &px, &tl);
+                                const long long nt = (c->nface[dX] + px - 1) / px;
+                                for (long long tt = 0; tt < 2 * nt; ++tt)
+                                    flow[gi].push_back({N, {arg, 0, tt}});
+                                for (long long tt = 0; tt < nt; ++tt)
+                                    curl[gi].push_back({N, {arg, 0, tt}});
+                                lean_cells[gi] += double(c->ncell);
+                                for (int w = 0; w < 2; ++w)
+                                    lean_lds[gi][w] = std::max(lean_lds[gi][w],
+                                                               mag_lean_lds(w, dX, N, px, es));
+                                continue;
+                            }
                             const MagTile& mt = c->mtile[dX];
                             mag_cells += double(c->ncell);
                             long long ntile = (c->nface[dX] + mt.PX - 1) / mt.PX;
@@ -510,6 +552,18 @@ static int build_plans(imh_batch* b) {
                         std::vector<BatchTile> tl = sorted(g.tl);
                         add_launch(p, f, tl);
                     }
+                    for (int gi = 0; gi < 6; ++gi)
+                        for (int w = 0; w < 2 && !flow[gi].empty(); ++w) {
+                            Launch m{};
+                            m.kind = w == 0 ? L_MAG_FLOW : L_MAG_CURL;
+                            m.lane = 0;  // simulations with a magnetic field
+                            m.d = gi / 2;
+                            m.general = gi & 1;
+                            m.smem = lean_lds[gi][w];
+                            m.bytes = (w == 0 ? 8.0 : 7.0) * lean_cells[gi] * es;
+                            std::vector<BatchTile> tl = sorted(w == 0 ? flow[gi] : curl[gi]);
+                            add_launch(p, m, tl);
+                        }
                     if (!adv[0].empty()) {
                         for (int s2 = 0; s2 < 2; ++s2) {
                             Launch a1{};
@@ -596,6 +650,11 @@ static hipError_t run_launch(imh_batch* b, const Launch& L, hipStream_t st) {
     case L_MAG_CT:
         return launch_magnet_batch<T>(1, (const MagnetArgs<T>*)b->margs, tl, L.ntiles, nb, L.kmax,
                                       L.smem, st);
+    case L_MAG_FLOW:
+    case L_MAG_CURL:
+        return launch_magnet_lean<T>(L.kind == L_MAG_FLOW ? 0 : 1,
+                                     (const MagnetLeanArgs<T>*)b->mlargs, tl, L.ntiles, nb, L.d,
+                                     L.general, L.smem, st);
     case L_CELLMAG:
         return launch_cell_centered_batch<T>((const CellMagArgs<T>*)b->cargs, tl, L.ntiles, nb, st);
     case L_END: return launch_end_iteration(b->sims_dev, n, st);

@@ -63,7 +63,7 @@ struct imh_ctx {
     int active_lin[3];
     hipStream_t st = nullptr;
     void* f[IMH_NFIELDS] = {};
-    void* scratch = nullptr;        // mag(I).flux(X) for the CT step
+    void* scratch = nullptr;        // mag(I).flux(X) for the CT steps, both components
     double* edges = nullptr;
     size_t edges_len = 0;
     size_t edges_cap = 0;               // doubles allocated at edges (>= edges_len)
@@ -203,6 +203,11 @@ template <typename T>
 imh::FluidArgs<T> make_fluid_args(const imh_ctx* c, int d, int force);
 template <typename T>
 imh::MagnetArgs<T> make_magnet_args(const imh_ctx* c, int dX, int dI, int force);
+void mag_lean_tile(const imh_ctx* c, int d, int* px, int* tl);
+bool magnet_lean_tracked(const imh_ctx* c);
+bool magnet_lean_ok(const imh_ctx* c, int dX, const int I[2]);
+template <typename T>
+imh::MagnetLeanArgs<T> make_magnet_lean_args(const imh_ctx* c, int dX, const int I[2], int force);
 template <typename T>
 imh::CellMagArgs<T> make_cellmag_args(const imh_ctx* c, int k, int force);
 template <typename T>

@@ -103,6 +103,22 @@ __device__ __forceinline__ int xcd_round_tile(int r, int ntiles) {
     return t < hi ? t : -1;
 }
 
+// The (argument block, tile) a block works on in round t of a persistent launch; with
+// tiles == nullptr the launch is one simulation, args[0], one block per tile.
+__device__ inline bool next_tile(const BatchTile* tiles, int ntiles, int r, int& arg,
+                                 long long& tile) {
+    if (!tiles) {
+        if (r > 0 || (int)blockIdx.x >= ntiles) return false;
+        arg = 0;
+        tile = xcd_tile(blockIdx.x, ntiles);  // neighbouring tiles on one XCD
+        return true;
+    }
+    const int t = xcd_round_tile(r, ntiles);
+    if (t < 0) return false;
+    uniform_tile(tiles, t, arg, tile);
+    return true;
+}
+
 // The general form of the sweep (fluid_sweep_impl.h).
 template <typename T>
 hipError_t launch_fluid_batch(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
@@ -180,6 +196,56 @@ struct MagnetArgs {
 };
 
 
+// One magnetFlux(X, [I1 I2]) of one simulation in the lean form (magnet_lean_impl.h): both
+// components' advection, then both CT steps and the cell-centred updates.
+template <typename T>
+struct MagnetLeanArgs {
+    const T* rho;            // mass
+    const T* mom;            // mom(X)
+    T* bI[2];                // mag(I1), mag(I2)
+    T* bX;                   // mag(X)
+    T* cI;                   // cell-centred mag(I2) and mag(X)
+    T* cX;
+    T* flux;                 // scratch: the limited fluxes of I1, then of I2 (ncell each)
+    double* edges;
+    const long long* eoff;
+    const SimDev* sim;
+    int n0, n1, n2;
+    int dI[2];
+    int ndims;
+    int modes;               // packed BC modes
+    int active_linX, active_linI[2];
+    int limiter;
+    double dxX, dxI[2];
+    int PX, TL;              // tile: PX pencils x TL threads, powers of two
+    long long npencil, ncell;
+    int bc_inf;
+    int force;
+};
+constexpr int MLEAN_BS = 256;
+// which = 0: advection, 2 tiles (I1, I2) per pencil group; 1: CT, one.  trk: some boundary
+// of the grid is transparent or a wall (magnet_lean_tracked).  lds: mag_lean_lds
+// of the launch's largest tile.
+template <typename T>
+hipError_t launch_magnet_lean(int which, const MagnetLeanArgs<T>* args, const BatchTile* tiles,
+                              int ntiles, int nblocks, int d, bool trk, size_t lds,
+                              hipStream_t st);
+template <>
+hipError_t launch_magnet_lean<double>(int, const MagnetLeanArgs<double>*, const BatchTile*, int,
+                                      int, int, bool, size_t, hipStream_t);
+template <>
+hipError_t launch_magnet_lean<float>(int, const MagnetLeanArgs<float>*, const BatchTile*, int, int,
+                                     int, bool, size_t, hipStream_t);
+
+// LDS of a tile.  Advection: two rows per pencil of N + 8 values (x rows padded by one value
+// in four, mlean::pad); CT: one row of N.
+__host__ __device__ constexpr int mag_lean_row(bool x, int N) {
+    return x ? (N + 8) + ((N + 8) >> 2) + 1 : N + 8;
+}
+inline size_t mag_lean_lds(int which, int d, int N, int PX, size_t esz) {
+    return which == 0 ? 2 * esz * PX * mag_lean_row(d == 0, N) : esz * PX * N;
+}
+
 // updateCellCentered for component k: cmag_k = 0.5*(B_k + shift_k(B_k, +1)).
 template <typename T>
 struct CellMagArgs {
@@ -242,8 +308,7 @@ constexpr int LANE1D_KMAX = LANE1D_NMAX / LANE1D_BS;
 template <typename T>
 struct Lane1dArgs {
     FluidArgs<T> fa;        // the sweep along x
-    MagnetArgs<T> ma[3];    // [dI] for X = x (dI = 1, 2)
-    CellMagArgs<T> ca[3];   // [k]
+    MagnetLeanArgs<T> ml[2];  // magnetFlux(X=1), I = [2 3] and [3 2]
 };
 hipError_t launch_lane1d(const void* args, int nsims, hipStream_t st);
 

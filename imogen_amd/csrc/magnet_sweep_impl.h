@@ -692,24 +692,6 @@ __device__ __forceinline__ void cell_centered_body(const CellMagArgs<T>& ap, lon
     if (cell < ncell) cell_centered_cell(a, cell);
 }
 
-// Persistent batched forms: blocks walk a tile list spanning many simulations.
-// tiles == nullptr: the single simulation args[0], one block per tile.
-// The (argument block, tile) a block works on in round t of a persistent launch; with
-// tiles == nullptr the launch is one simulation, args[0], one block per tile.
-__device__ inline bool next_tile(const BatchTile* tiles, int ntiles, int r, int& arg,
-                                 long long& tile) {
-    if (!tiles) {
-        if (r > 0 || (int)blockIdx.x >= ntiles) return false;
-        arg = 0;
-        tile = xcd_tile(blockIdx.x, ntiles);  // neighbouring tiles on one XCD
-        return true;
-    }
-    const int t = xcd_round_tile(r, ntiles);
-    if (t < 0) return false;
-    uniform_tile(tiles, t, arg, tile);
-    return true;
-}
-
 // Persistent batched forms: blocks walk a tile list spanning many simulations (one call
 // site of each body: they are large).
 template <typename T, int KMAX>
