@@ -4,12 +4,11 @@
 // A batch is a view over simulation contexts (imh_ctx) sharing one HIP stream.  One
 // iteration of every simulation is a fixed sequence of launches:
 //
-//   begin  -> CFL reset / CFL reduction (tiles = (sim, cell chunk)) / dt finalize
+//   time update (tiles = (sim, cell chunk)): CFL reduction, dt, iteration counters
 //   for order in (+1, -1), for sweep slot t = 0..2, op o = 0..1:
 //       fluid sweeps      one persistent launch per (block size, KMAX, MHD) group over the
 //                         pencil tiles of every simulation whose op (t, o) is a fluid sweep
-//       magnet sweeps     advection and CT launches per component, then cell-centred B
-//   end    -> iteration counters
+//       magnet sweeps     advection and CT launches
 //
 // Every simulation keeps its own sweep order (flux.m: the perms row follows its own
 // iteration number), so the launch plan repeats with period 6 in the batch step; the six
@@ -39,15 +38,15 @@ using namespace imh;
 
 namespace {
 
-enum LaunchKind { L_BEGIN, L_CFL_RESET, L_CFL, L_FINALIZE, L_FLUID, L_MAG_ADV, L_MAG_CT, L_CELLMAG,
-                  L_MAG_FLOW, L_MAG_CURL, L_END,
+enum LaunchKind { L_CFL, L_CFL_FINISH, L_FLUID, L_MAG_ADV, L_MAG_CT, L_CELLMAG,
+                  L_MAG_FLOW, L_MAG_CURL,
                   L_FORK, L_JOIN, L_SOURCE, L_LANE1D };
 
 constexpr int MAX_LANES = 2;
 
 struct Launch {
     LaunchKind kind;
-    int step;       // finalize: 1 or 2; source: the simulation
+    int step;       // CFL: 1 or 2; source: the simulation
     int bs, kmax;   // fluid / magnet variant
     bool mhd;
     bool general;   // fluid: the general kernel form, else the lean one; lean magnet: tracked
@@ -57,7 +56,6 @@ struct Launch {
     int ntiles;
     double bytes;   // algorithmic HBM bytes of the launch
     int lane;       // -1: the batch stream; else the lane's stream
-    bool reset;     // begin: also clear the CFL slots (the reduction follows)
 };
 
 int launch_kind_class(LaunchKind k) {
@@ -368,39 +366,33 @@ static int build_plans(imh_batch* b) {
     if (b->nlanes == 1)
         for (int i = 0; i < n; ++i) lane[i] = 0;
     for (int p = 0; p < 6; ++p) {
-        Launch L{};
-        L.lane = -1;
         std::vector<BatchTile> none;
-        L.kind = L_BEGIN;
-        L.reset = true;  // the first CFL reduction follows
-        add_launch(p, L, none);
         auto cfl_block = [&](int step) {
             std::vector<BatchTile> tl;
             double by = 0;
+            bool several = false;  // a simulation of several tiles
             for (int i = 0; i < n; ++i) {
                 const imh_ctx* c = b->ctx[i];
-                long long nch = (c->ncell + cfl_chunk() - 1) / cfl_chunk();
+                const long long chunk = cfl_chunk(c->ncell), nch = (c->ncell + chunk - 1) / chunk;
+                several = several || nch > 1;
                 for (long long t = 0; t < nch; ++t) tl.push_back({i, 0, t});
                 int nf = 5;
                 for (int k = 0; k < 3; ++k) nf += c->mag_is_zero[k] ? 0 : 1;
                 by += double(nf) * c->ncell * es;
             }
-            if (step > 1) {  // the begin launch cleared the slots for step 1
-                Launch r{};
-                r.kind = L_CFL_RESET;
-                r.lane = -1;
-                add_launch(p, r, none);
-            }
             Launch c{};
             c.kind = L_CFL;
             c.lane = -1;
+            c.step = step;
             c.bytes = by;
             add_launch(p, c, tl);
-            Launch f{};
-            f.kind = L_FINALIZE;
-            f.lane = -1;
-            f.step = step;
-            add_launch(p, f, none);
+            if (several) {
+                Launch f{};
+                f.kind = L_CFL_FINISH;
+                f.lane = -1;
+                f.step = step;
+                add_launch(p, f, none);
+            }
         };
         auto fork_join = [&](LaunchKind k) {
             if (b->nlanes < 2) return;
@@ -603,10 +595,6 @@ static int build_plans(imh_batch* b) {
             }
         }
         fork_join(L_JOIN);
-        Launch E{};
-        E.lane = -1;
-        E.kind = L_END;
-        add_launch(p, E, none);
     }
     if (all.size() > b->tiles_cap) {
         hipFree(b->tiles);
@@ -631,10 +619,12 @@ static hipError_t run_launch(imh_batch* b, const Launch& L, hipStream_t st) {
     // a multiple of 8 blocks: the XCD-range schedule (xcd_round_tile)
     const int nb = ((std::max(1, std::min(L.ntiles, b->ncu * 4)) + 7) / 8) * 8;
     switch (L.kind) {
-    case L_BEGIN: return launch_begin_iteration(b->sims_dev, b->pars_dev, n, 0, st, L.reset ? 1 : 0);
-    case L_CFL_RESET: return launch_cfl_reset(b->sims_dev, n, st);
-    case L_CFL: return launch_cfl_batch<T>((const CflArgs<T>*)b->cflargs, tl, L.ntiles, nb, st);
-    case L_FINALIZE: return launch_time_finalize(b->sims_dev, b->pars_dev, n, L.step, st);
+    case L_CFL:
+        return launch_cfl<T>((const CflArgs<T>*)b->cflargs, tl, L.ntiles, nb,
+                             L.step == 1 ? CFL_RUNNING : CFL_ACTIVE, L.step, 1, st);
+    case L_CFL_FINISH:
+        return launch_cfl_finish<T>((const CflArgs<T>*)b->cflargs, n,
+                                    L.step == 1 ? CFL_RUNNING : CFL_ACTIVE, L.step, 1, st);
     case L_FLUID:
         if (L.bs == 0)
             return launch_fluid_column<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.mhd,
@@ -657,7 +647,6 @@ static hipError_t run_launch(imh_batch* b, const Launch& L, hipStream_t st) {
                                      L.general, L.smem, st);
     case L_CELLMAG:
         return launch_cell_centered_batch<T>((const CellMagArgs<T>*)b->cargs, tl, L.ntiles, nb, st);
-    case L_END: return launch_end_iteration(b->sims_dev, n, st);
     case L_SOURCE: return imh_launch_source(b->ctx[L.step], st);
     case L_LANE1D: return launch_lane1d(b->l1args, (int)b->fused_list.size(), st);
     case L_FORK:

@@ -1,11 +1,21 @@
-// cfl.hip -- CFL timestep reduction (time/TimeManager.m:55-99), device-side time
+// cfl.hip -- CFL timestep reduction (time/TimeManager.m:55-99) with the device-side time
 // bookkeeping, and the compensated conservation totals.
 //
-// The CFL maximum of |p_i/rho| + c_s for i = 1..3 is reduced per block with wavefront
-// shuffles and one LDS pass, then merged with one 64-bit atomicMax per block and
-// direction (non-negative doubles order like their bit patterns).  dt is computed on the
+// Two launches per time update: every block reduces |p_i/rho| + c_s, i = 1..3, over its cells
+// (16-byte loads of four consecutive cells, wavefront shuffles, one LDS pass) and stores its
+// three maxima; a block per simulation then reduces those, computes dt and advances time and
+// iteration.  A simulation of one tile (up to 4096 cells) is finished by the first launch.
+// Whether a simulation runs at all both evaluate from its time state.  dt is computed on the
 // device, so an iteration needs no host round trip and can be replayed as a hipGraph.
+//
+// Bound by HBM on large grids, by FP64 issue on FP32 fields: one reciprocal of rho serves
+// its four quotients (LMath: rounded as the divisions are).  CFL reduction, us, against one
+// cell per load and three 64-bit atomics per block on the same addresses: FP64 125^3 45 -> 21,
+// 512^2 25 -> 11, FP32 1024^2 37 -> 14, 192^3 78 -> 34 (141 MB).  The loop body's bookkeeping
+// launches: 4 -> 1, or none up to 4096 cells.  Finding the last block by a ticket instead of a
+// second launch loses (1024^2 38 us, 256^3 186: each block's release and acquire).
 #include "imh_common.h"
+#include "fluid_lean_impl.h"
 #include "imh_host.h"
 #include "imh_kernels.h"
 
@@ -18,74 +28,94 @@ __device__ inline double wave_max(double v) {
     return v;
 }
 
-__device__ inline void atomic_max_nonneg(unsigned long long* slot, double v) {
-    if (!(v >= 0.0)) return;  // NaN: MATLAB max ignores it
-    atomicMax(slot, (unsigned long long)__double_as_longlong(v));
+constexpr int CFL_BS = 256;
+
+// Maxima of m over the block in every thread (NaN ignored: MATLAB max; 0 when all are NaN).
+__device__ __forceinline__ void block_max(double (&m)[3], double (*s_red)[CFL_BS / 64]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double v = wave_max(m[k]);
+        if (lane == 0) s_red[k][wave] = v;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const double v = fmax(fmax(s_red[k][0], s_red[k][1]), fmax(s_red[k][2], s_red[k][3]));
+        m[k] = v >= 0.0 ? v : 0.0;
+    }
+}
+
+// |p_i/rho| + c_s (pressure.m 'sound', the operations of pressure_sound) of one cell.
+__device__ __forceinline__ void cell_speeds(double rho, double px, double py, double pz, double E,
+                                            double bx, double by, double bz, const MagUse& u,
+                                            double g, double (&m)[3]) {
+    using M = LMath<double>;
+    const double inv = M::rcp(rho);
+    const double v2 = M::quot(px * px + py * py + pz * pz, rho * rho);
+    double b2 = 0.0;
+    if (u.x) b2 = 0.0 + bx * bx;
+    if (u.y) b2 = b2 + by * by;
+    if (u.z) b2 = b2 + bz * bz;
+    double r = (g - 1.0) * (E - 0.5 * rho * v2);
+    r = r - (g - 1.0) * 0.5 * b2;
+    const double cs = M::root(fabs(M::div(g * r + 2.0 * b2, rho, inv)));
+    m[0] = fmax(m[0], fabs(M::div(px, rho, inv)) + cs);
+    m[1] = fmax(m[1], fabs(M::div(py, rho, inv)) + cs);
+    m[2] = fmax(m[2], fabs(M::div(pz, rho, inv)) + cs);
 }
 
 }  // namespace
 
-// Max of |p_i/rho| + c_s over cells [c0, c1) of one simulation (grid-strided by
-// `stride`), merged into the simulation's slots with one atomic per block and direction.
+// The speeds of cells [c0, c1), c0 a multiple of 4, into m.
 template <typename T>
-__device__ __forceinline__ void cfl_body(const CflArgs<T>& a, long long c0, long long c1,
-                                         long long stride) {
-    __shared__ double s_red[3][4];
-    if (!a.sim->active) return;
-    double m[3] = {NAN, NAN, NAN};
-    // U cells per thread and round, every load of the round issued before any use (a
-    // loop of one cell at a time waits a memory round trip per cell); cells past c1 read
-    // cell c0 and are left out of the maxima
-    constexpr int U = 4;
-    for (long long cb = c0 + threadIdx.x; cb < c1; cb += stride * U) {
-        T q[5][U], b[3][U];
+__device__ __forceinline__ void cfl_cells(const CflArgs<T>& a, long long c0, long long c1,
+                                          double (&m)[3]) {
+    typedef T V4 __attribute__((ext_vector_type(4)));
+    for (long long c = c0 + 4 * threadIdx.x; c < c1; c += 4 * CFL_BS) {
+        T q[5][4], b[3][4];
+        if (c + 4 <= c1) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const long long c = cb + u * stride < c1 ? cb + u * stride : c0;
+            for (int v = 0; v < 5; ++v) {
+                const V4 x = *(const IMH_GLOBAL_AS V4*)(gmem(a.q[v]) + c);
 #pragma unroll
-            for (int v = 0; v < 5; ++v) q[v][u] = gmem(a.q[v])[c];
+                for (int u = 0; u < 4; ++u) q[v][u] = x[u];
+            }
 #pragma unroll
-            for (int k = 0; k < 3; ++k) b[k][u] = a.bc[k] ? gmem(a.bc[k])[c] : T(0);
+            for (int k = 0; k < 3; ++k) {
+                V4 x = {T(0), T(0), T(0), T(0)};
+                if (a.bc[k]) x = *(const IMH_GLOBAL_AS V4*)(gmem(a.bc[k]) + c);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) b[k][u] = x[u];
+            }
+        } else {  // the last cells, the first of them again in place of those past c1
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const long long cu = c + u < c1 ? c + u : c;
+#pragma unroll
+                for (int v = 0; v < 5; ++v) q[v][u] = gmem(a.q[v])[cu];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) b[k][u] = a.bc[k] ? gmem(a.bc[k])[cu] : T(0);
+            }
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (cb + u * stride >= c1) continue;
-            const double rho = double(q[0][u]);
-            const double px = double(q[1][u]), py = double(q[2][u]), pz = double(q[3][u]);
-            const double cs = pressure_sound(rho, px, py, pz, double(q[4][u]), double(b[0][u]),
-                                             double(b[1][u]), double(b[2][u]), a.use, a.gamma);
-            m[0] = fmax(m[0], fabs(px / rho) + cs);
-            m[1] = fmax(m[1], fabs(py / rho) + cs);
-            m[2] = fmax(m[2], fabs(pz / rho) + cs);
-        }
+        for (int u = 0; u < 4; ++u)
+            cell_speeds(double(q[0][u]), double(q[1][u]), double(q[2][u]), double(q[3][u]),
+                        double(q[4][u]), double(b[0][u]), double(b[1][u]), double(b[2][u]), a.use,
+                        a.gamma, m);
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int k = 0; k < 3; ++k) {
-        double v = wave_max(m[k]);
-        if (lane == 0) s_red[k][wave] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x < 3) {
-        int k = threadIdx.x;
-        double v = fmax(fmax(s_red[k][0], s_red[k][1]), fmax(s_red[k][2], s_red[k][3]));
-        atomic_max_nonneg(&a.sim->cmax_bits[k], v);
-    }
-    __syncthreads();
 }
 
-constexpr long long CFL_CHUNK = 256 * 32;  // cells per tile of a batched launch
-
-// dt of one simulation from its reduced speeds cmax_bits[3] (TimeManager.m:65-98).
-__device__ inline void finalize_sim(SimDev& d, const SimParams& q, int step,
-                                    const unsigned long long (&cmax_bits)[3]) {
-    if (!d.active) return;
-    if (step > 1 && q.update_mode != 0) return;
-    double cmax = 1e-2;
+// dt of one simulation from its reduced speeds (TimeManager.m:65-98).
+__device__ inline void finalize_sim(SimDev& d, const SimParams& q, const double (&speed)[3]) {
+    double cmax = 1e-2, dx = 0.0;
     int gi = 0;
+#pragma unroll
     for (int k = 0; k < 3; ++k) {
-        double c = __longlong_as_double((long long)cmax_bits[k]);
-        if (c > cmax) {
-            cmax = c;
+        if (speed[k] > cmax) {
+            cmax = speed[k];
+            dx = q.dgrid[k];
             gi = k + 1;
         }
     }
@@ -96,7 +126,7 @@ __device__ inline void finalize_sim(SimDev& d, const SimParams& q, int step,
     }
     d.grid_index = gi;
     double upd = double(q.update_mode + 1);
-    d.dt = q.cfl * q.dgrid[gi - 1] / cmax;
+    d.dt = q.cfl * dx / cmax;
     double newtime = d.time + upd * d.dt;
     if (newtime > q.time_max) {
         d.dt = (q.time_max - d.time) / upd;
@@ -105,100 +135,133 @@ __device__ inline void finalize_sim(SimDev& d, const SimParams& q, int step,
     d.time = newtime;
 }
 
+// TimeManager.running (TimeManager.m:36-39), evaluated at the top of the loop body.
+__device__ inline int running(const SimDev& d, const SimParams& q) {
+    return (d.iteration <= q.iter_max) && (d.time < q.time_max) && d.error == 0;
+}
+
+// Whether a simulation takes part in time update `step` (2: only with update_mode 0).
+__device__ inline int cfl_runs(const SimDev& d, const SimParams& par, int gate, int step) {
+    if (step > 1 && par.update_mode != 0) return -1;  // no second update
+    return gate == CFL_ALWAYS ? 1 : (gate == CFL_ACTIVE ? d.active : running(d, par));
+}
+
+// The end of a time update, by one thread.  count: the loop body's iteration = iteration + 1
+// (TimeManager.step) goes with its last time update; nothing reads it in between.
+__device__ inline void cfl_finish(SimDev& d, const SimParams& par, int run, int gate, int step,
+                                  int count, const double (&m)[3]) {
+    if (gate != CFL_ACTIVE) d.active = run;
+    if (!run) return;
+    finalize_sim(d, par, m);
+    if (count && d.active && step == (par.update_mode == 0 ? 2 : 1)) d.iteration += 1;
+}
+
 template <typename T>
-__global__ void __launch_bounds__(256) cfl_batch_kernel(const CflArgs<T>* args,
-                                                        const BatchTile* tiles, int ntiles) {
+__global__ void __launch_bounds__(CFL_BS) cfl_kernel(const CflArgs<T>* args, const BatchTile* tiles,
+                                                     int ntiles, int gate, int step, int count) {
+    __shared__ double s_red[3][CFL_BS / 64];
     for (int r = 0;; ++r) {
-        const int t = tiles ? xcd_round_tile(r, ntiles) : int(blockIdx.x + r * gridDim.x);
-        if (t < 0 || t >= ntiles) break;
+        const BatchTile* tl = tiles;
+        asm volatile("" : "+s"(tl));  // opaque: one copy of the body serves both forms
         int arg = 0;
-        long long tile = t;
-        if (tiles) uniform_tile(tiles, t, arg, tile);
-        const CflArgs<T> a = args[arg];  // private copy, read once per tile
-        long long c0 = tile * a.chunk;
-        long long c1 = c0 + a.chunk < a.ncell ? c0 + a.chunk : a.ncell;
-        cfl_body(a, c0, c1, 256);
+        long long tile;
+        if (tl) {
+            const int t = xcd_round_tile(r, ntiles);
+            if (t < 0) break;
+            uniform_tile(tl, t, arg, tile);
+        } else {
+            if (r > 0 || (int)blockIdx.x >= ntiles) break;
+            tile = blockIdx.x;
+        }
+        const CflArgs<T> a = uniform_load(&args[arg]);
+        const SimParams par = uniform_load(a.par);
+        const int run = cfl_runs(*a.sim, par, gate, step);
+        double m[3] = {NAN, NAN, NAN};
+        if (run > 0) {
+            const long long c0 = tile * a.chunk;
+            cfl_cells(a, c0, c0 + a.chunk < a.ncell ? c0 + a.chunk : a.ncell, m);
+            block_max(m, s_red);
+        }
+        if (a.chunk >= a.ncell) {
+            __syncthreads();  // every thread has read the time state
+            if (run >= 0 && threadIdx.x == 0) cfl_finish(*a.sim, par, run, gate, step, count, m);
+        } else if (run > 0 && threadIdx.x == 0) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) gmem(a.part)[3 * tile + k] = m[k];
+        }
+        __syncthreads();
     }
 }
 
+// The second launch: block s finishes simulation s (of those with several tiles).
 template <typename T>
-hipError_t launch_cfl_batch(const CflArgs<T>* args, const BatchTile* tiles, int ntiles,
-                            int nblocks, hipStream_t st) {
+__global__ void __launch_bounds__(CFL_BS) cfl_finish_kernel(const CflArgs<T>* args, int gate,
+                                                            int step, int count) {
+    __shared__ double s_red[3][CFL_BS / 64];
+    const CflArgs<T> a = uniform_load(&args[blockIdx.x]);
+    if (a.chunk >= a.ncell) return;
+    const SimParams par = uniform_load(a.par);
+    const int run = cfl_runs(*a.sim, par, gate, step);
+    if (run < 0) return;
+    double m[3] = {NAN, NAN, NAN};
+    if (run) {
+        const int ntile = int((a.ncell + a.chunk - 1) / a.chunk);
+        for (int t = threadIdx.x; t < ntile; t += CFL_BS)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) m[k] = fmax(m[k], gmem(a.part)[3 * t + k]);
+    }
+    block_max(m, s_red);
+    if (threadIdx.x == 0) cfl_finish(*a.sim, par, run, gate, step, count, m);
+}
+
+template <typename T>
+hipError_t launch_cfl(const CflArgs<T>* args, const BatchTile* tiles, int ntiles, int nblocks,
+                      int gate, int step, int count, hipStream_t st) {
     if (ntiles == 0) return hipSuccess;
-    hipLaunchKernelGGL((cfl_batch_kernel<T>), dim3(nblocks), dim3(256), 0, st, args, tiles, ntiles);
+    hipLaunchKernelGGL((cfl_kernel<T>), dim3(nblocks), dim3(CFL_BS), 0, st, args, tiles, ntiles,
+                       gate, step, count);
+    return hipGetLastError();
+}
+template <typename T>
+hipError_t launch_cfl_finish(const CflArgs<T>* args, int nsims, int gate, int step, int count,
+                             hipStream_t st) {
+    hipLaunchKernelGGL((cfl_finish_kernel<T>), dim3(nsims), dim3(CFL_BS), 0, st, args, gate, step,
+                       count);
     return hipGetLastError();
 }
 
-template hipError_t launch_cfl_batch<double>(const CflArgs<double>*, const BatchTile*, int, int,
-                                             hipStream_t);
-template hipError_t launch_cfl_batch<float>(const CflArgs<float>*, const BatchTile*, int, int,
-                                            hipStream_t);
+template hipError_t launch_cfl<double>(const CflArgs<double>*, const BatchTile*, int, int, int, int,
+                                       int, hipStream_t);
+template hipError_t launch_cfl<float>(const CflArgs<float>*, const BatchTile*, int, int, int, int,
+                                      int, hipStream_t);
+template hipError_t launch_cfl_finish<double>(const CflArgs<double>*, int, int, int, int,
+                                              hipStream_t);
+template hipError_t launch_cfl_finish<float>(const CflArgs<float>*, int, int, int, int, hipStream_t);
 
-long long cfl_chunk() { return CFL_CHUNK; }
+// Cells per tile: a whole simulation of up to 4096; else at most CFL_TILES tiles of a
+// multiple of four cells per thread.
+long long cfl_chunk(long long ncell) {
+    const long long per = 4LL * CFL_BS;
+    if (ncell <= 4 * per) return 4 * per;
+    return per * ((ncell + per * CFL_TILES - 1) / (per * CFL_TILES));
+}
 
-// The kernels below run one thread per simulation over arrays of per-simulation
-// pointers (a batch is a view over independently allocated simulations).
-
-// TimeManager.running (TimeManager.m:36-39), evaluated at the top of the loop body.
-// reset: also clear the CFL slots of the active simulations (the reset before the CFL
-// reduction, done here when that reduction follows).
+// The top of the loop body on its own (direct calls of parts of it), one thread per
+// simulation over an array of per-simulation pointers.
 __global__ void begin_iteration_kernel(SimDev* const* sim, const SimParams* const* p, int nsims,
-                                       int unconditional, int reset) {
+                                       int unconditional) {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nsims) return;
     SimDev& d = *sim[s];
-    const SimParams& q = *p[s];
-    int running = (d.iteration <= q.iter_max) && (d.time < q.time_max) && d.error == 0;
-    d.active = (unconditional || running) ? 1 : 0;
-    if (reset && d.active)
-        for (int k = 0; k < 3; ++k) d.cmax_bits[k] = 0ull;
-}
-
-__global__ void cfl_reset_kernel(SimDev* const* sim, int nsims) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsims) return;
-    SimDev& d = *sim[s];
-    if (!d.active) return;
-    for (int k = 0; k < 3; ++k) d.cmax_bits[k] = 0ull;
-}
-
-// dt from the reduced speeds (TimeManager.m:65-98).
-__global__ void time_finalize_kernel(SimDev* const* sim, const SimParams* const* p, int nsims,
-                                     int step) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsims) return;
-    SimDev& d = *sim[s];
-    const unsigned long long cm[3] = {d.cmax_bits[0], d.cmax_bits[1], d.cmax_bits[2]};
-    finalize_sim(d, *p[s], step, cm);
-}
-
-// TimeManager.step: iteration = iteration + 1.
-__global__ void end_iteration_kernel(SimDev* const* sim, int nsims) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsims) return;
-    if (sim[s]->active) sim[s]->iteration += 1;
+    d.active = (unconditional || running(d, *p[s])) ? 1 : 0;
 }
 
 static inline int nblk(int n) { return (n + 255) / 256; }
 
 hipError_t launch_begin_iteration(SimDev* const* sim, const SimParams* const* p, int nsims,
-                                  int unconditional, hipStream_t st, int reset) {
+                                  int unconditional, hipStream_t st) {
     hipLaunchKernelGGL(begin_iteration_kernel, dim3(nblk(nsims)), dim3(256), 0, st, sim, p, nsims,
-                       unconditional, reset);
-    return hipGetLastError();
-}
-hipError_t launch_cfl_reset(SimDev* const* sim, int nsims, hipStream_t st) {
-    hipLaunchKernelGGL(cfl_reset_kernel, dim3(nblk(nsims)), dim3(256), 0, st, sim, nsims);
-    return hipGetLastError();
-}
-hipError_t launch_time_finalize(SimDev* const* sim, const SimParams* const* p, int nsims,
-                                int step, hipStream_t st) {
-    hipLaunchKernelGGL(time_finalize_kernel, dim3(nblk(nsims)), dim3(256), 0, st, sim, p, nsims,
-                       step);
-    return hipGetLastError();
-}
-hipError_t launch_end_iteration(SimDev* const* sim, int nsims, hipStream_t st) {
-    hipLaunchKernelGGL(end_iteration_kernel, dim3(nblk(nsims)), dim3(256), 0, st, sim, nsims);
+                       unconditional);
     return hipGetLastError();
 }
 

@@ -415,13 +415,16 @@ static long long edges_layout(const imh_config& cfg, long long eoff[NOBJ][2][3])
 
 static void layout_edges(imh_ctx* c) { c->edges_len = (size_t)edges_layout(c->cfg, c->eoff); }
 
+// Partial sums of the conservation totals (8 fields); the CFL maxima of the tiles follow.
+constexpr size_t CSUM_PART = 2 * 1024 * 8;
+
 // Device bytes of a context (fields, CT scratch, edge stores, small bookkeeping).
 static size_t ctx_bytes(const imh_config& cfg, size_t edges_len) {
     const size_t es = cfg.precision == IMH_FP64 ? 8 : 4;
     const size_t ncell = (size_t)cfg.grid[0] * cfg.grid[1] * cfg.grid[2];
     size_t b = ncell * es * (IMH_NFIELDS + (cfg.magnet_active ? 2 : 0));
     b += edges_len * sizeof(double) + sizeof(long long) * NOBJ * 6 + 2 * sizeof(SimDev);
-    b += ARG_SLOT * ARG_RING + 6 * ARG_SLOT * CAP_SLOTS + sizeof(double) * (2 * 1024 * 8 + 8) +
+    b += ARG_SLOT * ARG_RING + 6 * ARG_SLOT * CAP_SLOTS + sizeof(double) * (CSUM_PART + 3 * CFL_TILES + 8) +
          sizeof(double) * MAX_FADE;
     return b;
 }
@@ -484,7 +487,7 @@ static int ctx_alloc(imh_ctx* c) {
     CHK(hipMalloc(&c->par_ptr, sizeof(SimParams*)), "hipMalloc(par_ptr)");
     CHK(hipMemcpy(c->sim_ptr, &c->sim, sizeof(SimDev*), hipMemcpyHostToDevice), "sim_ptr");
     CHK(hipMemcpy(c->par_ptr, &c->par, sizeof(SimParams*), hipMemcpyHostToDevice), "par_ptr");
-    CHK(hipMalloc(&c->csum_part, sizeof(double) * 2 * 1024 * 8), "hipMalloc(csum)");
+    CHK(hipMalloc(&c->csum_part, sizeof(double) * (CSUM_PART + 3 * CFL_TILES)), "hipMalloc(csum)");
     CHK(hipMalloc(&c->csum_out, sizeof(double) * 8), "hipMalloc(csum_out)");
     CHK(hipHostMalloc((void**)&c->arg_host, ARG_SLOT * ARG_RING, hipHostMallocDefault),
         "hipHostMalloc(args)");
@@ -1169,7 +1172,9 @@ CflArgs<T> make_cfl_args(const imh_ctx* c) {
         a.bc[k] = c->mag_is_zero[k] ? nullptr : (const T*)c->f[IMH_F_CMAGX + k];
     a.sim = c->sim;
     a.ncell = c->ncell;
-    a.chunk = cfl_chunk();
+    a.par = c->par;
+    a.part = c->csum_part + CSUM_PART;
+    a.chunk = cfl_chunk(c->ncell);
     a.use = {!c->mag_is_zero[0], !c->mag_is_zero[1], !c->mag_is_zero[2]};
     a.gamma = c->cfg.gamma;
     return a;
@@ -1178,35 +1183,30 @@ template CflArgs<double> make_cfl_args<double>(const imh_ctx*);
 template CflArgs<float> make_cfl_args<float>(const imh_ctx*);
 
 template <typename T>
-static int cfl_t(imh_ctx* c) {
-    CflArgs<T> a = make_cfl_args<T>(c);
-    // one simulation: at most 2048 tiles of a multiple of 256 cells
-    a.chunk = ((c->ncell + 2048LL * 256 - 1) / (2048LL * 256)) * 256;
-    const void* da = imh_stage_args(c, &a, sizeof(a));
+static int cfl_t(imh_ctx* c, int gate, int step, int count) {
+    const CflArgs<T> a = make_cfl_args<T>(c);
+    const CflArgs<T>* da = (const CflArgs<T>*)imh_stage_args(c, &a, sizeof(a));
     if (!da) return IMH_EHIP;
     const int nt = int((c->ncell + a.chunk - 1) / a.chunk);
     int nb = 5;
     for (int k = 0; k < 3; ++k) nb += a.bc[k] ? 1 : 0;
-    ProfScope ps(c, IMH_K_CFL, double(nb) * c->ncell * sizeof(T));
-    hipError_t e = launch_cfl_batch((const CflArgs<T>*)da, nullptr, nt, nt, c->st);
+    hipError_t e;
+    {
+        ProfScope ps(c, IMH_K_CFL, double(nb) * c->ncell * sizeof(T));
+        e = launch_cfl(da, nullptr, nt, nt, gate, step, count, c->st);
+    }
+    if (e == hipSuccess && nt > 1) {
+        ProfScope ps(c, IMH_K_BOOK, 0.0);
+        e = launch_cfl_finish(da, 1, gate, step, count, c->st);
+    }
     return e == hipSuccess ? IMH_OK : hip_fail(e, "cfl launch");
 }
 
-int imh_time_update_internal(imh_ctx* c, int step) {
+// TimeManager.update; gate: CFL_ALWAYS / CFL_RUNNING / CFL_ACTIVE; count: part of a loop body.
+int imh_time_update_internal(imh_ctx* c, int step, int gate, int count) {
     if (step > 1 && c->cfg.update_mode != 0) return IMH_OK;  // TimeManager.m:61-63
-    hipError_t e;
-    {
-        ProfScope ps(c, IMH_K_BOOK, 0.0);
-        e = launch_cfl_reset(c->sim_ptr, 1, c->st);
-    }
-    if (e != hipSuccess) return hip_fail(e, "cfl reset");
-    int rc = c->cfg.precision == IMH_FP64 ? cfl_t<double>(c) : cfl_t<float>(c);
-    if (rc) return rc;
-    {
-        ProfScope ps(c, IMH_K_BOOK, 0.0);
-        e = launch_time_finalize(c->sim_ptr, c->par_ptr, 1, step, c->st);
-    }
-    return e == hipSuccess ? IMH_OK : hip_fail(e, "time finalize");
+    return c->cfg.precision == IMH_FP64 ? cfl_t<double>(c, gate, step, count)
+                                        : cfl_t<float>(c, gate, step, count);
 }
 
 int imh_flux_internal(imh_ctx* c, int order, int force) {
@@ -1293,24 +1293,15 @@ int imh_source_internal(imh_ctx* c) {
 // One imogen.m:61-71 loop body; `conditional` = 0 runs it unconditionally (imh_iteration).
 int imh_iteration_body(imh_ctx* c, int conditional) {
     int rc;
-    hipError_t e;
-    {
-        ProfScope ps(c, IMH_K_BOOK, 0.0);
-        e = launch_begin_iteration(c->sim_ptr, c->par_ptr, 1, conditional ? 0 : 1, c->st);
-    }
-    if (e != hipSuccess) return hip_fail(e, "begin iteration");
     for (int i = 1; i <= 2; ++i) {
-        if ((rc = imh_time_update_internal(c, i))) return rc;
+        // the first update also evaluates TimeManager.running, the last counts the iteration
+        const int gate = i == 2 ? CFL_ACTIVE : (conditional ? CFL_RUNNING : CFL_ALWAYS);
+        if ((rc = imh_time_update_internal(c, i, gate, 1))) return rc;
         if ((rc = imh_flux_internal(c, i == 1 ? 1 : -1, 0))) return rc;
         // treadmill: inactive; gravity.solvePotential: the fixed potential is set once;
         // source(): without gravity and radiation, ener - dt*0 changes no value
         if ((rc = imh_source_internal(c))) return rc;
     }
-    {
-        ProfScope ps(c, IMH_K_BOOK, 0.0);
-        e = launch_end_iteration(c->sim_ptr, 1, c->st);
-    }
-    if (e != hipSuccess) return hip_fail(e, "end iteration");
     return IMH_OK;
 }
 
@@ -1332,7 +1323,7 @@ int imh_time_update(imh_ctx* c, int step) {
     // a direct call behaves as inside an unconditional loop body
     hipError_t e = launch_begin_iteration(c->sim_ptr, c->par_ptr, 1, 1, c->st);
     if (e != hipSuccess) return hip_fail(e, "begin");
-    return imh_time_update_internal(c, step);
+    return imh_time_update_internal(c, step, CFL_ACTIVE, 0);
 }
 
 int imh_flux(imh_ctx* c, int order) {

@@ -43,7 +43,7 @@ enum FluxType : int { FT_OTHER = 0, FT_FLUXL = 1, FT_FLUXR = 2, FT_FLUX = 3 };
 struct SimDev {
     double dt;                 // run.time.dTime
     double time;               // run.time.time
-    unsigned long long cmax_bits[3];  // max(|p_i/rho| + c_s) as ordered bits (>= 0)
+    double spare[3];
     int iteration;             // run.time.iteration
     int grid_index;            // last CFL direction
     int error;                 // IMH_ECFL when no speed exceeds 1e-2

@@ -195,7 +195,7 @@ hipError_t launch_edges_from_field(const void* field, bool fp64, const int n[3],
 // internal entry points (force = run regardless of the loop's running flag)
 int imh_fluid_sweep_internal(imh_ctx* c, int X, int force);
 int imh_magnet_sweep_internal(imh_ctx* c, int X, const int I[2], int force);
-int imh_time_update_internal(imh_ctx* c, int step);
+int imh_time_update_internal(imh_ctx* c, int step, int gate, int count);
 int imh_flux_internal(imh_ctx* c, int order, int force);
 
 // argument blocks of one simulation (imh_api.cpp), shared with the batched path

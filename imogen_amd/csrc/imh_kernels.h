@@ -329,25 +329,31 @@ struct CflArgs {
     const T* q[5];
     const T* bc[3];
     SimDev* sim;
+    const SimParams* par;
+    double* part;            // the tiles' maxima, 3 * CFL_TILES
     long long ncell;
-    long long chunk;         // cells per tile (a multiple of 256)
+    long long chunk;         // cells per tile (cfl_chunk)
     MagUse use;
     double gamma;
 };
 
+constexpr int CFL_TILES = 1024;  // most tiles of one simulation
+// gate: whether a simulation runs: always, when TimeManager.running holds (both set its
+// active flag), or by that flag.
+constexpr int CFL_ALWAYS = 0, CFL_RUNNING = 1, CFL_ACTIVE = 2;
 template <typename T>
-hipError_t launch_cfl_batch(const CflArgs<T>* args, const BatchTile* tiles, int ntiles,
-                            int nblocks, hipStream_t st);
-long long cfl_chunk();
+hipError_t launch_cfl(const CflArgs<T>* args, const BatchTile* tiles, int ntiles, int nblocks,
+                      int gate, int step, int count, hipStream_t st);
+// After launch_cfl, where a simulation has several tiles (chunk < ncell).
+template <typename T>
+hipError_t launch_cfl_finish(const CflArgs<T>* args, int nsims, int gate, int step, int count,
+                             hipStream_t st);
+long long cfl_chunk(long long ncell);
 
-// Device-side bookkeeping kernels (cfl.hip), one thread per simulation; `sim` and `p`
+// The top of the loop body on its own (cfl.hip), one thread per simulation; `sim` and `p`
 // are device arrays of per-simulation pointers.
 hipError_t launch_begin_iteration(SimDev* const* sim, const SimParams* const* p, int nsims,
-                                  int unconditional, hipStream_t st, int reset = 0);
-hipError_t launch_cfl_reset(SimDev* const* sim, int nsims, hipStream_t st);
-hipError_t launch_time_finalize(SimDev* const* sim, const SimParams* const* p, int nsims,
-                                int step, hipStream_t st);
-hipError_t launch_end_iteration(SimDev* const* sim, int nsims, hipStream_t st);
+                                  int unconditional, hipStream_t st);
 
 // Conservation totals (Neumaier-compensated FP64, fixed-order tree).
 template <typename T>

@@ -15,8 +15,14 @@
 //                         cell-centred B_X.
 // The general form takes six launches, and its y / z pencils read one cell per row; here
 // the lanes of y / z tiles run over adjacent pencils.  A tile is PX whole pencils, so that
-// B_I and B_X can be updated in place.  What bounds it: memory latency and L2 bandwidth (the
-// arithmetic is some 100 instructions per cell and component).
+// B_I and B_X can be updated in place.  What bounds it: HBM and L2 traffic on large grids (FP64
+// 200^3: 150 us of advection and 107 of CT for 512 and 448 MB), the latency of a tile's chain
+// (loads, LDS, windows, stores) on small ones; the arithmetic is some 100 instructions per
+// cell and component.  Per magnetFlux call, general -> lean: FP64 100^3 85 -> 32 us, 512^2 52 ->
+// 16 (x) and 22 (y); the 1-D lane's iteration (lane1d.hip) 181 -> 130.
+//
+// TRK: some boundary is transparent or a wall.  Without, the kernels hold no tracker code: FP64
+// advection 147 -> 88 vector registers (3 -> 5 waves per SIMD), CT 89 -> 57.
 //
 // Past a pencil end the windows hold the wrapped cells (circular) or the ghosts of each
 // shift call in the .m text's order, from the object's edge tracker (other modes), put in by

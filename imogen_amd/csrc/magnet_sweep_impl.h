@@ -1,7 +1,9 @@
 // magnet_sweep_impl.h -- constrained-transport magnetic sweep (magnet/magnetFlux.m,
 // magnet/relaxingMagnet.m, MagnetArray.updateCellCentered).
 //
-// One magnetFlux(X, [I1 I2]) call is, per component I:
+// The general form: first assignments, fade ends, spacing lines, pencils below 8 cells, a
+// circular end opposite another mode (magnet_lean_impl.h takes the rest).  One
+// magnetFlux(X, [I1 I2]) call is, per component I:
 //   magnet_advect_kernel  (pencils along X): grid-aligned velocity (shift of mass and
 //                         mom(X) along I, smoothing along X), upwind predictor, TVD
 //                         corrector with the limiter, B_I update; the limited flux is kept
