@@ -51,6 +51,7 @@ struct Launch {
     bool mhd;
     bool general;   // fluid: the general kernel form, else the lean one; lean magnet: tracked
     int d, px;      // lean forms: sweep dimension; fluid: most pencils of a tile
+    int form;       // fluid, lean form: lean_form
     size_t smem;
     long long off;  // into the tile array
     int ntiles;
@@ -423,12 +424,13 @@ static int build_plans(imh_batch* b) {
             }
             for (int t = 0; t < 3; ++t)
                 for (int o = 0; o < 2; ++o) {
-                    // fluid groups keyed by (bs, kmax, mhd, general, and d in the lean form)
+                    // fluid groups keyed by (bs, kmax, mhd, general, and d and form in the lean form)
                     struct G {
                         int lane;
                         int bs, kmax;
                         bool mhd, general;
                         int d, px;
+                        int form;
                         double bytes;
                         std::vector<std::pair<int, BatchTile>> tl;
                     };
@@ -453,21 +455,25 @@ static int build_plans(imh_batch* b) {
                         if (fluid_op && c->cfg.fluid_active) {
                             const int dX = X - 1;
                             bool gen = c->cfg.bc[0][dX] == IMH_BC_FADE ||
-                                       c->cfg.bc[1][dX] == IMH_BC_FADE || c->visc_type ||
+                                       c->cfg.bc[1][dX] == IMH_BC_FADE || c->visc_type == 2 ||
                                        c->dline_dev[dX];
                             const FluidTile& ft = fluid_tile(c, dX, gen);
                             // bs 0: the column march (one thread per pencil)
-                            const bool col = ft.column && !gen;
+                            const bool col = ft.column && !gen && !c->visc_type;
                             if (!col && ft.PX > LEAN_PXMAX) gen = true;
                             const int gbs = col ? 0 : ft.bs, gkm = col ? 0 : ft.kmax;
                             const int gd = (col || gen) ? 0 : dX;
+                            const int form = (col || gen) ? 0 : lean_form(c->visc_type, c->cfg.bc[0][dX],
+                                                                          c->cfg.bc[1][dX]);
                             G* g = nullptr;
                             for (G& gg : groups)
                                 if (gg.lane == lane[i] && gg.bs == gbs && gg.kmax == gkm &&
-                                    gg.mhd == c->mhd_kernel && gg.general == gen && gg.d == gd)
+                                    gg.mhd == c->mhd_kernel && gg.general == gen && gg.d == gd &&
+                                    gg.form == form)
                                     g = &gg;
                             if (!g) {
-                                groups.push_back({lane[i], gbs, gkm, c->mhd_kernel, gen, gd, 1, 0.0, {}});
+                                groups.push_back({lane[i], gbs, gkm, c->mhd_kernel, gen, gd, 1, form,
+                                                  0.0, {}});
                                 g = &groups.back();
                             }
                             g->px = std::max(g->px, ft.PX);
@@ -540,6 +546,7 @@ static int build_plans(imh_batch* b) {
                         f.general = g.general;
                         f.d = g.d;
                         f.px = g.px;
+                        f.form = g.form;
                         f.bytes = g.bytes;
                         std::vector<BatchTile> tl = sorted(g.tl);
                         add_launch(p, f, tl);
@@ -633,7 +640,7 @@ static hipError_t run_launch(imh_batch* b, const Launch& L, hipStream_t st) {
             return launch_fluid_batch<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.bs,
                                          L.kmax, L.mhd, st);
         return launch_fluid_lean<T>((const FluidArgs<T>*)b->fargs, tl, L.ntiles, nb, L.bs, L.kmax,
-                                    L.d, L.mhd, L.px, st);
+                                    L.d, L.mhd, L.px, L.form, st);
     case L_MAG_ADV:
         return launch_magnet_batch<T>(0, (const MagnetArgs<T>*)b->margs, tl, L.ntiles, nb, L.kmax,
                                       L.smem, st);

@@ -23,22 +23,22 @@ template hipError_t launch_fluid_batch<float>(const FluidArgs<float>*, const Bat
 
 template <typename T>
 hipError_t launch_fluid_lean(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
-                             int nblocks, int bs, int kmax, int d, bool mhd, int px,
+                             int nblocks, int bs, int kmax, int d, bool mhd, int px, int form,
                              hipStream_t st) {
     if (ntiles == 0) return hipSuccess;
     constexpr int esz = (int)sizeof(T);
 #define IMH_LEAN_PICK(E, B, K)                                                           \
     if (esz == E && bs == B && kmax == K)                                                \
-        return IMH_LEAN_LAUNCHER(E, B, K)(args, tiles, ntiles, nblocks, d, mhd, px, st);
+        return IMH_LEAN_LAUNCHER(E, B, K)(args, tiles, ntiles, nblocks, d, mhd, px, form, st);
     IMH_FLUID_VARIANTS(IMH_LEAN_PICK)
 #undef IMH_LEAN_PICK
     return hipErrorInvalidValue;
 }
 
 template hipError_t launch_fluid_lean<double>(const FluidArgs<double>*, const BatchTile*, int, int,
-                                              int, int, int, bool, int, hipStream_t);
+                                              int, int, int, bool, int, int, hipStream_t);
 template hipError_t launch_fluid_lean<float>(const FluidArgs<float>*, const BatchTile*, int, int,
-                                             int, int, int, bool, int, hipStream_t);
+                                             int, int, int, bool, int, int, hipStream_t);
 
 bool fluid_variant_compiled(int esz, int bs, int kmax) {
 #define IMH_FLUID_HAS(E, B, K) \

@@ -1,6 +1,7 @@
 // fluid_lean_impl.h -- the fluid sweep (relaxingFluid.m:16-73, wFluidFlux.m:14-44,
-// pressure.m) of the common case: no fade end, no first assignment of the flux objects,
-// no viscosity, uniform spacing.  fluid_sweep_impl.h holds the general form.
+// pressure.m) of the common case: no fade end, no first assignment of the flux objects, no
+// Caramana-Shashkov-Whalen viscosity, uniform spacing.  fluid_sweep_impl.h holds the general
+// form.
 //
 // A workgroup owns PX whole pencils, TL = BS / PX threads each, K consecutive cells per
 // thread in registers.  What bounds a sweep here is not HBM but the latency of one tile
@@ -21,6 +22,11 @@
 //  * The argument block is read into scalar registers (uniform_load): FP64 4 cells per
 //    thread 168 vector registers with spills -> 147, 2 cells 123; FP64 256^3 664 -> 621 us per
 //    sweep, FP32 192^3 158 -> 147, a 1024-cell tube 18.0 -> 16.9.
+//  * Three kernels (FORM): without ghost jobs where both ends are circular or constant (FP64
+//    MHD, 2 cells per thread: 139 -> 120 vector registers; 100^3 47.5 -> 44.6 us per sweep, FP32
+//    MHD 191^2 13.2 -> 12.4), with them, and with Neumann-Richtmyer viscosity (the sweep momentum
+//    of the next chunk through two more LDS rows; FP64 96^3 with gravity and radiation 123 -> 43
+//    against the general form).
 // Measured against the general form (us per sweep, mean of the directions): FP64 125^3 175 ->
 // 78, 256^3 1463 -> 621 (1.34 GB: 2.2 TB/s), 333x333 19 -> 15, FP32 192^3 372 -> 147,
 // 1024x1024 37 -> 26, FP64 MHD 96^3 61 -> 43.  Spilling registers for one more wave per SIMD
@@ -145,16 +151,18 @@ constexpr int PXMAX = LEAN_PXMAX;   // pencils per tile
 
 // Dynamic LDS of a block: byte offsets of its parts and its size.  The 20 exchange rows
 // hold one value per thread and, per pencil, the value past each end (lower, upper).
+// With viscosity, two more rows: the sweep momentum of each chunk's first and last cell.
 struct Lds {
-    int trk, red, ends, total;
+    int trk, red, ends, visc, total;
 };
 __host__ __device__ constexpr int row_len(int bs) { return bs + 2 * PXMAX; }
-__host__ __device__ constexpr Lds lds_layout(int bs, int px, int esz) {
+__host__ __device__ constexpr Lds lds_layout(int bs, int px, int esz, bool visc = false) {
     Lds L{};
     L.trk = 20 * row_len(bs) * esz;
     L.red = L.trk + px * 30 * 8;                  // edge trackers [job][3], FP64
     L.ends = L.red + 2 * (bs / 64) * px * esz;    // pencil maxima per wave, 2 stages
-    L.total = L.ends + px * 40 * esz;             // [side][field][cell from the end][2]
+    L.visc = L.ends + px * 40 * esz;              // (ends: [side][field][cell from the end][2])
+    L.total = L.visc + (visc ? 2 * bs * esz : 0);
     return L;
 }
 
@@ -240,12 +248,13 @@ __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, doubl
 }  // namespace lean
 
 // The sweep of one tile (PX pencils) of one simulation along D.  lds: lean::lds_layout.
-template <typename T, int BS, int K, bool MHD, int D>
+template <typename T, int BS, int K, bool MHD, int D, int FORM = LEAN_ENDS>
 __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long long tile, char* lds) {
     const FluidArgs<T> a = uniform_load(&ap);
     if (!a.force && !uniform_load(&a.sim->active)) return;
     using M = LMath<T>;
     constexpr bool XM = D == 0;
+    constexpr bool VISC = FORM == LEAN_VISC;
     constexpr int X = D + 1;
     constexpr int NW = BS / 64;
     constexpr int RL = lean::row_len(BS);
@@ -307,8 +316,8 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     const double g = a.gamma;
     const int mlo = mode_at(a.modes, 0, D), mhi = mode_at(a.modes, 1, D);
     // circular and constant ends take their ghosts from the exchange rows
-    const bool simple = (mlo == IMH_BC_CIRC || mlo == IMH_BC_CONST) &&
-                        (mhi == IMH_BC_CIRC || mhi == IMH_BC_CONST);
+    const bool simple = FORM == LEAN_PLAIN ||
+                        (lean_plain_end(mlo) && lean_plain_end(mhi));
     const int ty_last = (N - 1) / K;
     const bool own_lo = ty == 0, own_hi = ty == ty_last;   // chunk with cell 0 / cell N-1
     // where the neighbouring chunks' values are read: past a pencil end, the other end's
@@ -391,8 +400,46 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     // Numerators of wFluidFlux.m (w = numerator / C) of state Q into nu, and the largest
     // |u| + c of the chunk.
     T nu[5][K];
-    auto numerators = [&](const T (&Q)[5][K]) __attribute__((always_inline)) -> T {
+    auto numerators = [&](const T (&Q)[5][K], int obj) __attribute__((always_inline)) -> T {
         T lmax = T(NAN);
+        // Neumann-Richtmyer viscosity (ArtificialViscosity.m:73-77): vm = min(p(i+1) - p(i), 0)
+        // of the sweep momentum, whose objects are obj + X (the FluidArray in the predictor,
+        // its StorageArray in the corrector); press gains vm .* (c1 .* c_f + c2 .* vm ./ rho)
+        T vm[K];
+        if constexpr (VISC) {
+            T* const s_mv = reinterpret_cast<T*>(lds + L.visc);
+            s_mv[tid] = Q[X][0];
+            s_mv[BS + tid] = Q[X][K - 1];
+            __syncthreads();
+            T nb = Q[X][K - 1];
+            if (ty < ty_last) nb = s_mv[tid + dstep];
+            if (own_hi) {
+                T c0 = Q[X][0], c1 = s_mv[BS + (ty > 0 ? tid - dstep : tid)];
+#pragma unroll
+                for (int k = 1; k < K; ++k)
+                    if (i0 + k < N) {
+                        c1 = c0;
+                        c0 = Q[X][k];
+                    }
+                if (mhi == IMH_BC_CIRC) {
+                    nb = s_mv[t_first];
+                } else {
+                    const bool trk = pen_ok && (mhi == IMH_BC_TRANS || mhi == IMH_BC_WALL);
+                    double tv = 0.0;
+                    IMH_GLOBAL_AS double* const tp =
+                        gmem(a.edges) + (trk ? a.eoff[((obj + X) * 2 + 1) * 3 + D] + pface : 0);
+                    if (trk) tv = *tp;
+                    nb = T(lean::end_ghost(mhi, true, false, double(c0), double(c1), a.active_lin,
+                                           a.bc_inf, tv));
+                    if (trk && mhi == IMH_BC_TRANS) *tp = tv;
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const T up = (k + 1 < K && i0 + k < N - 1) ? Q[X][k + 1 < K ? k + 1 : k] : nb;
+                vm[k] = fmin(up - Q[X][k], T(0));  // MATLAB min(.., 0) skips NaN
+            }
+        }
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             const T bx = MHD ? bm[0][k] : T(0), by = MHD ? bm[1][k] : T(0),
@@ -403,6 +450,13 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
             const T sp = fabs(U) + c;
             lmax = fmax(lmax, sp);  // NaN-ignoring, like MATLAB max
             nu[0][k] = Q[X][k];
+            if constexpr (VISC) {
+                const T t = T(a.visc_quad) * vm[k];
+                T tr;
+                if constexpr (sizeof(T) == 8) tr = M::divrho2(t, Q[0][k], ir);
+                else tr = t / Q[0][k];
+                P = P + vm[k] * (T(a.visc_lin) * c + tr);
+            }
             if constexpr (MHD) {
                 const T bX = sel3(D, bx, by, bz);
                 const T b[3] = {bx, by, bz};
@@ -548,7 +602,7 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     };
 
     // ================= predictor: W and C from U^n (wFluidFlux.m) ====================
-    publish_max(0, numerators(q));
+    publish_max(0, numerators(q, OBJ_PRIM));
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
         row(v * 4 + 0)[tid] = q[v][0];
@@ -612,7 +666,7 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
 
     // ================= corrector: W' and C' from U^(n+1/2) ===========================
     {
-        const T m = numerators(q);
+        const T m = numerators(q, OBJ_FSTORE);
         publish_max(1, i0 < N ? m : T(NAN));
     }
     __syncthreads();  // also: every thread has read the predictor's rows
@@ -745,7 +799,7 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
 
 #ifdef IMH_LEAN_OCCUPANCY
 // Persistent batched form (tiles != nullptr) or one block per tile of args[0].
-template <typename T, int BS, int K, bool MHD, int D>
+template <typename T, int BS, int K, bool MHD, int D, int FORM>
 __global__ void __launch_bounds__(BS) IMH_LEAN_OCCUPANCY
 fluid_lean_kernel(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles) {
     extern __shared__ __attribute__((aligned(16))) char lean_lds[];
@@ -763,7 +817,7 @@ fluid_lean_kernel(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles) 
             if (r > 0 || (int)blockIdx.x >= ntiles) break;
             tile = args[0].xcd_remap ? xcd_tile(blockIdx.x, ntiles) : (long long)blockIdx.x;
         }
-        fluid_lean_body<T, BS, K, MHD, D>(args[arg], tile, lean_lds);
+        fluid_lean_body<T, BS, K, MHD, D, FORM>(args[arg], tile, lean_lds);
         __syncthreads();
     }
 }

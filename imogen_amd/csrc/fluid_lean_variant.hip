@@ -21,13 +21,14 @@ using LeanT = float;
 
 hipError_t IMH_LEAN_LAUNCHER(IMH_FLUID_ESZ, IMH_FLUID_BS, IMH_FLUID_KMAX)(
     const void* args, const BatchTile* tiles, int ntiles, int nblocks, int d, bool mhd,
-    int px, hipStream_t st) {
+    int px, int form, hipStream_t st) {
     if (px > lean::PXMAX) return hipErrorInvalidValue;
     const FluidArgs<LeanT>* a = (const FluidArgs<LeanT>*)args;
-    const size_t lds = (size_t)lean::lds_layout(IMH_FLUID_BS, px, IMH_FLUID_ESZ).total;
-#define IMH_LL(M, DD)                                                                       \
-    if (mhd == M && d == DD) {                                                              \
-        auto* fn = fluid_lean_kernel<LeanT, IMH_FLUID_BS, IMH_FLUID_KMAX, M, DD>;             \
+    const size_t lds =
+        (size_t)lean::lds_layout(IMH_FLUID_BS, px, IMH_FLUID_ESZ, form == LEAN_VISC).total;
+#define IMH_LL(M, DD, F)                                                                    \
+    if (mhd == M && d == DD && form == F) {                                                 \
+        auto* fn = fluid_lean_kernel<LeanT, IMH_FLUID_BS, IMH_FLUID_KMAX, M, DD, F>;          \
         if (lds > 64 * 1024) {                                                              \
             hipError_t e = hipFuncSetAttribute((const void*)fn,                             \
                                                hipFuncAttributeMaxDynamicSharedMemorySize,  \
@@ -37,8 +38,11 @@ hipError_t IMH_LEAN_LAUNCHER(IMH_FLUID_ESZ, IMH_FLUID_BS, IMH_FLUID_KMAX)(
         hipLaunchKernelGGL(fn, dim3(nblocks), dim3(IMH_FLUID_BS), lds, st, a, tiles, ntiles); \
         return hipGetLastError();                                                           \
     }
-    IMH_LL(false, 0) IMH_LL(false, 1) IMH_LL(false, 2) IMH_LL(true, 0) IMH_LL(true, 1)
-    IMH_LL(true, 2)
+#define IMH_LF(F) \
+    IMH_LL(false, 0, F) IMH_LL(false, 1, F) IMH_LL(false, 2, F) IMH_LL(true, 0, F) \
+    IMH_LL(true, 1, F) IMH_LL(true, 2, F)
+    IMH_LF(LEAN_PLAIN) IMH_LF(LEAN_ENDS) IMH_LF(LEAN_VISC)
+#undef IMH_LF
 #undef IMH_LL
     return hipErrorInvalidValue;
 }

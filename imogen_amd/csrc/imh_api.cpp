@@ -937,13 +937,15 @@ static int fluid_sweep_t(imh_ctx* c, int d, int force) {
     hipError_t e;
     if (long_sweep(c, d)) {
         e = launch_fluid_long<T>(a, c->long_scratch, c->ncell, c->mhd_kernel, c->st);
-    } else if (t.column && !general) {
+    } else if (t.column && !general && !a.visc_type) {
         const int nt = int((a.npencil + fluid_column_pencils() - 1) / fluid_column_pencils());
         e = launch_fluid_column((const FluidArgs<T>*)da, nullptr, nt, nt, c->mhd_kernel, c->st);
     } else if (!general && t.PX <= LEAN_PXMAX) {
         const int nt = int((a.npencil + t.PX - 1) / t.PX);
         e = launch_fluid_lean((const FluidArgs<T>*)da, nullptr, nt, nt, t.bs, t.kmax, d,
-                              c->mhd_kernel, t.PX, c->st);
+                              c->mhd_kernel, t.PX,
+                              lean_form(a.visc_type, mode_at(a.modes, 0, d), mode_at(a.modes, 1, d)),
+                              c->st);
     } else {
         const int nt = int((a.npencil + t.PX - 1) / t.PX);
         e = launch_fluid_batch((const FluidArgs<T>*)da, nullptr, nt, nt, t.bs, t.kmax,

@@ -124,11 +124,21 @@ template <typename T>
 hipError_t launch_fluid_batch(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
                               int nblocks, int bs, int kmax, bool mhd, hipStream_t st);
 constexpr int LEAN_PXMAX = 16;   // pencils per tile of the lean sweep
+// Kernels of the lean sweep: both ends circular or constant (no ghost jobs), any ends, and any
+// ends with Neumann-Richtmyer viscosity.
+constexpr int LEAN_PLAIN = 0, LEAN_ENDS = 1, LEAN_VISC = 2;
+__host__ __device__ constexpr bool lean_plain_end(int mode) {
+    return mode == IMH_BC_CIRC || mode == IMH_BC_CONST;
+}
+inline int lean_form(int visc_type, int mlo, int mhi) {
+    if (visc_type) return LEAN_VISC;
+    return lean_plain_end(mlo) && lean_plain_end(mhi) ? LEAN_PLAIN : LEAN_ENDS;
+}
 // The lean form (fluid_lean_impl.h) of a sweep along d that fluid_needs_general() does not
-// send to the general form; px: the most pencils a tile of the launch holds.
+// send to the general form; px: the most pencils a tile of the launch holds; form: lean_form.
 template <typename T>
 hipError_t launch_fluid_lean(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
-                             int nblocks, int bs, int kmax, int d, bool mhd, int px,
+                             int nblocks, int bs, int kmax, int d, bool mhd, int px, int form,
                              hipStream_t st);
 // The column march for sweeps along y / z with circular or constant boundaries: one
 // thread per pencil, fluid_column_pencils() pencils per tile.
@@ -138,10 +148,10 @@ hipError_t launch_fluid_column(const FluidArgs<T>* args, const BatchTile* tiles,
 int fluid_column_pencils();
 
 // whether a sweep of these arguments needs the general kernel form: the first sweep of a
-// simulation, a fade boundary, viscosity or a spacing line
+// simulation, a fade boundary, Caramana-Shashkov-Whalen viscosity or a spacing line
 template <typename T>
 inline bool fluid_needs_general(const FluidArgs<T>& a) {
-    return a.init_edges || a.visc_type || a.dxl || mode_at(a.modes, 0, a.d) == IMH_BC_FADE ||
+    return a.init_edges || a.visc_type == 2 || a.dxl || mode_at(a.modes, 0, a.d) == IMH_BC_FADE ||
            mode_at(a.modes, 1, a.d) == IMH_BC_FADE;
 }
 
@@ -162,7 +172,8 @@ IMH_FLUID_VARIANTS(IMH_FLUID_DECLARE)
 #define IMH_LEAN_LAUNCHER(E, B, K) IMH_LEAN_LAUNCHER_(E, B, K)
 #define IMH_LEAN_DECLARE(E, B, K)                                                          \
     hipError_t IMH_LEAN_LAUNCHER(E, B, K)(const void* args, const BatchTile* tiles, int ntiles, \
-                                          int nblocks, int d, bool mhd, int px, hipStream_t st);
+                                          int nblocks, int d, bool mhd, int px, int form,   \
+                                          hipStream_t st);
 IMH_FLUID_VARIANTS(IMH_LEAN_DECLARE)
 bool fluid_variant_compiled(int esz, int bs, int kmax);
 

@@ -85,3 +85,24 @@ def test_fp32(grid, magnet):
             assert rel_l1(b.download(f), ref) <= 1e-5, f
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("bc", ["circ", "trans", "wall", "mirror", ["const", "flip"], ["trans", "zero"]])
+@pytest.mark.parametrize("magnet", [False, True])
+def test_neumann_richtmyer(bc, magnet):
+    """The viscosity's shifted momentum at chunk ends, and its upper ghost in every mode;
+    pencils whose last chunk holds one to four cells."""
+    for n, tile in [(3, None), (9, (256, 4, 16)), (10, (256, 4, 8)), (23, (256, 2, 4)), (259, None)]:
+        ini, st = box((n, 5, 1) if n > 100 else (n, 6, 4), {"x": bc, "y": bc, "z": bc}, "vanleer",
+                      magnet, seed=n)
+        orc, run = make_oracle(ini, st), make_gpu(ini, st)
+        orc.set_viscosity("neumann_richtmyer", 0.2, 0.4)
+        run.set_viscosity("neumann_richtmyer", 0.2, 0.4)
+        if tile:
+            run.set_fluid_tile(1, *tile)
+        for _ in range(3):
+            orc.iteration()
+            iteration(run)
+            compare(run, orc, FLUID_FIELDS + (MAG_FIELDS if magnet else []), TOL)
+        run.close()
+        orc.close()
