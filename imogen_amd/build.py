@@ -32,6 +32,7 @@ VARIANT_SRC = "fluid_sweep_variant.hip"
 LEAN_VARIANT_SRC = "fluid_lean_variant.hip"
 MAG_VARIANT_SRC = "magnet_sweep_variant.hip"
 MAG_LEAN_SRC = "magnet_lean_variant.hip"
+LINE_SRC = "line1d_variant.hip"
 
 
 def fluid_variants():
@@ -65,6 +66,8 @@ def units():
         out.append((LEAN_VARIANT_SRC, "fluid_lean_v%d_%d_%d" % (e, b, k), list(out[-1][2])))
     for e in (8, 4):
         out.append((MAG_LEAN_SRC, "magnet_lean_v%d" % e, ["-DIMH_MAG_ESZ=%d" % e] + (fp32 if e == 4 else [])))
+    for e in (8, 4):
+        out.append((LINE_SRC, "line1d_v%d" % e, ["-DIMH_LINE_ESZ=%d" % e] + (fp32 if e == 4 else [])))
     for e, k in magnet_variants():
         out.append((MAG_VARIANT_SRC, "magnet_sweep_v%d_%d" % (e, k),
                     ["-DIMH_MAG_ESZ=%d" % e, "-DIMH_MAG_KMAX=%d" % k] + (fp32 if e == 4 else [])))
@@ -107,7 +110,7 @@ def build(verbose=False, jobs=None, incremental=False, out=None, defines=()):
     os.makedirs(build_dir, exist_ok=True)
     us = units()
     # the long fluid variants first, so they overlap with the short units
-    us.sort(key=lambda u: 0 if u[0] in (VARIANT_SRC, LEAN_VARIANT_SRC, MAG_LEAN_SRC, MAG_VARIANT_SRC) else 1)
+    us.sort(key=lambda u: 0 if u[0] in (VARIANT_SRC, LEAN_VARIANT_SRC, MAG_LEAN_SRC, LINE_SRC, MAG_VARIANT_SRC) else 1)
     jobs = jobs or min(len(us), max(1, (os.cpu_count() or 2)))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
         results = list(ex.map(lambda u: _compile(u, verbose, incremental, defines, build_dir), us))

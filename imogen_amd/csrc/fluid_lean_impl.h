@@ -247,11 +247,12 @@ __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, doubl
 
 }  // namespace lean
 
-// The sweep of one tile (PX pencils) of one simulation along D.  lds: lean::lds_layout.
+// The sweep of one tile (PX pencils) of one simulation along D.  lds: lean::lds_layout; dt:
+// the same for all lanes.
 template <typename T, int BS, int K, bool MHD, int D, int FORM = LEAN_ENDS>
-__device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long long tile, char* lds) {
+__device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long long tile, char* lds,
+                                                double dt) {
     const FluidArgs<T> a = uniform_load(&ap);
-    if (!a.force && !uniform_load(&a.sim->active)) return;
     using M = LMath<T>;
     constexpr bool XM = D == 0;
     constexpr bool VISC = FORM == LEAN_VISC;
@@ -310,7 +311,6 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
         return base + unsigned(i) * stride;
     };
 
-    const double dt = uniform_load(&a.sim->dt);
     const double ff = dt / a.dx;          // fluxFactor = dTime ./ DGRID{X}
     const double hf = 0.5 * ff;
     const double g = a.gamma;
@@ -817,7 +817,9 @@ fluid_lean_kernel(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles) 
             if (r > 0 || (int)blockIdx.x >= ntiles) break;
             tile = args[0].xcd_remap ? xcd_tile(blockIdx.x, ntiles) : (long long)blockIdx.x;
         }
-        fluid_lean_body<T, BS, K, MHD, D, FORM>(args[arg], tile, lean_lds);
+        double dt;
+        if (sweep_runs(args[arg], dt))
+            fluid_lean_body<T, BS, K, MHD, D, FORM>(args[arg], tile, lean_lds, dt);
         __syncthreads();
     }
 }

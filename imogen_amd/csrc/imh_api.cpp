@@ -1307,6 +1307,55 @@ int imh_iteration_body(imh_ctx* c, int conditional) {
     return IMH_OK;
 }
 
+// Whether the loop body of a 1-D simulation can run in the one-workgroup kernel
+// (line1d_variant.hip): lean sweeps only, no source terms, no viscosity.
+static bool line1d_ok(const imh_ctx* c) {
+    const imh_config& g = c->cfg;
+    if (c->n[1] != 1 || c->n[2] != 1 || c->n[0] < 3 || c->n[0] > LINE1D_NMAX) return false;
+    if (!g.fluid_active || !c->fluid_init || c->grav || c->rad_type || c->visc_type ||
+        c->dline_dev[0] || long_sweep(c, 0))
+        return false;
+    for (int s = 0; s < 2; ++s)
+        if (g.bc[s][0] == IMH_BC_FADE || g.bc[s][0] == IMH_BC_WORMHOLE) return false;
+    if (!g.magnet_active) return true;
+    for (int it = 0; it < 6; ++it)
+        for (int o = 0; o < 2; ++o) {  // the same component order in every iteration
+            int dirs[3], mi[3][2];
+            sweep_order(it + 1, o ? -1 : 1, g.perms_order, dirs, mi);
+            for (int t = 0; t < 3; ++t)
+                if (dirs[t] == 1 && (mi[t][0] != (o ? 3 : 2) || !magnet_lean_ok(c, 0, mi[t])))
+                    return false;
+        }
+    return true;
+}
+
+template <typename T>
+static int line1d_t(imh_ctx* c, int iterations) {
+    const int N = c->n[0];
+    FluidArgs<T> fa = make_fluid_args<T>(c, 0, 0);
+    fa.PX = 1;
+    fa.TL = LINE1D_BS;
+    fa.K = 1;
+    while (fa.K * LINE1D_BS < N) fa.K *= 2;
+    fa.xmajor = 1;
+    const FluidArgs<T>* dfa = (const FluidArgs<T>*)imh_stage_args(c, &fa, sizeof(fa));
+    const MagnetLeanArgs<T>* dml[2] = {nullptr, nullptr};
+    for (int o = 0; o < 2 && c->cfg.magnet_active; ++o) {
+        const int I[2] = {o ? 3 : 2, o ? 2 : 3};
+        MagnetLeanArgs<T> ml = make_magnet_lean_args<T>(c, 0, I, 0);
+        ml.PX = 1;
+        ml.TL = LINE1D_BS;
+        dml[o] = (const MagnetLeanArgs<T>*)imh_stage_args(c, &ml, sizeof(ml));
+        if (!dml[o]) return IMH_EHIP;
+    }
+    const CflArgs<T> ca = make_cfl_args<T>(c);
+    const CflArgs<T>* dca = (const CflArgs<T>*)imh_stage_args(c, &ca, sizeof(ca));
+    if (!dfa || !dca) return IMH_EHIP;
+    hipError_t e = launch_line1d<T>(dfa, dml, dca, N, c->mhd_kernel, c->cfg.magnet_active != 0,
+                                    iterations, c->st);
+    return e == hipSuccess ? IMH_OK : hip_fail(e, "1-D iterations launch");
+}
+
 extern "C" {
 
 int imh_fluid_sweep(imh_ctx* c, int X) {
@@ -1536,6 +1585,13 @@ int imh_run(imh_ctx* c, int max_iterations, int* done) {
         bool inited = c->fluid_init || !c->cfg.fluid_active;
         if (!inited || c->no_graphs) {
             if ((rc = imh_iteration_body(c, 1))) return rc;
+        } else if (line1d_ok(c)) {
+            // up to the next look at the time state in one launch
+            const int n = std::min(todo - it, 64 - (it & 63));
+            rc = c->cfg.precision == IMH_FP64 ? line1d_t<double>(c, n) : line1d_t<float>(c, n);
+            if (rc) return rc;
+            it += n - 1;
+            c->host_iteration += n - 1;
         } else {
             int row = ((c->host_iteration - 1) % 6 + 6) % 6;
             if (!c->graph[row]) {

@@ -119,6 +119,15 @@ __device__ inline bool next_tile(const BatchTile* tiles, int ntiles, int r, int&
     return true;
 }
 
+// Whether the sweep of an argument block runs, and its time step (the time state is that of
+// the launches before: no kernel that reads it so may change it).
+template <typename A>
+__device__ __forceinline__ bool sweep_runs(const A& a, double& dt) {
+    const SimDev* sim = uniform_load(&a.sim);
+    dt = uniform_load(&sim->dt);
+    return uniform_load(&a.force) || uniform_load(&sim->active);
+}
+
 // The general form of the sweep (fluid_sweep_impl.h).
 template <typename T>
 hipError_t launch_fluid_batch(const FluidArgs<T>* args, const BatchTile* tiles, int ntiles,
@@ -323,17 +332,6 @@ struct Lane1dArgs {
 };
 hipError_t launch_lane1d(const void* args, int nsims, hipStream_t st);
 
-// Compiled magnet variants X(element size, KMAX): each a translation unit with the
-// advection and CT kernels for pencils of up to KMAX * TL cells.
-#define IMH_MAG_VARIANTS(X) \
-    X(8, 1) X(8, 2) X(8, 4) X(8, 8) X(8, 16) X(4, 1) X(4, 2) X(4, 4) X(4, 8) X(4, 16)
-#define IMH_MAG_LAUNCHER_(E, K) launch_magnet_v##E##_##K
-#define IMH_MAG_LAUNCHER(E, K) IMH_MAG_LAUNCHER_(E, K)
-#define IMH_MAG_DECLARE(E, K)                                                               \
-    hipError_t IMH_MAG_LAUNCHER(E, K)(int which, const void* args, const BatchTile* tiles,  \
-                                      int ntiles, int nblocks, size_t smem, hipStream_t st);
-IMH_MAG_VARIANTS(IMH_MAG_DECLARE)
-
 // CFL reduction (TimeManager.update) over one simulation.
 template <typename T>
 struct CflArgs {
@@ -347,6 +345,33 @@ struct CflArgs {
     MagUse use;
     double gamma;
 };
+
+// Several iterations of one 1-D simulation in one launch (line1d_variant.hip): time update,
+// flux call and iteration count of a pencil of up to LINE1D_NMAX cells by one workgroup.  mag: the
+// magnetic sweeps too, with ml[0] / ml[1] magnetFlux(X=1) for order +1 / -1.  bs * k >= N.
+constexpr int LINE1D_BS = 512;
+constexpr int LINE1D_NMAX = 8 * LINE1D_BS;
+template <typename T>
+hipError_t launch_line1d(const FluidArgs<T>* fa, const MagnetLeanArgs<T>* const ml[2],
+                         const CflArgs<T>* ca, int N, bool mhd, bool mag, int iterations,
+                         hipStream_t st);
+template <>
+hipError_t launch_line1d<double>(const FluidArgs<double>*, const MagnetLeanArgs<double>* const[2],
+                                 const CflArgs<double>*, int, bool, bool, int, hipStream_t);
+template <>
+hipError_t launch_line1d<float>(const FluidArgs<float>*, const MagnetLeanArgs<float>* const[2],
+                                const CflArgs<float>*, int, bool, bool, int, hipStream_t);
+
+// Compiled magnet variants X(element size, KMAX): each a translation unit with the
+// advection and CT kernels for pencils of up to KMAX * TL cells.
+#define IMH_MAG_VARIANTS(X) \
+    X(8, 1) X(8, 2) X(8, 4) X(8, 8) X(8, 16) X(4, 1) X(4, 2) X(4, 4) X(4, 8) X(4, 16)
+#define IMH_MAG_LAUNCHER_(E, K) launch_magnet_v##E##_##K
+#define IMH_MAG_LAUNCHER(E, K) IMH_MAG_LAUNCHER_(E, K)
+#define IMH_MAG_DECLARE(E, K)                                                               \
+    hipError_t IMH_MAG_LAUNCHER(E, K)(int which, const void* args, const BatchTile* tiles,  \
+                                      int ntiles, int nblocks, size_t smem, hipStream_t st);
+IMH_MAG_VARIANTS(IMH_MAG_DECLARE)
 
 constexpr int CFL_TILES = 1024;  // most tiles of one simulation
 // gate: whether a simulation runs: always, when TimeManager.running holds (both set its

@@ -33,17 +33,19 @@ namespace {
 // instantiated for that many): a short pencil does not run the longest pencil's body.
 template <typename T, int KC>
 __device__ __forceinline__ void lane1d_run(const Lane1dArgs<T>& a, char* s_fluid, T* s_mag) {
+    double dt;
+    if (!sweep_runs(a.fa, dt)) return;
     // steps 0 and 3: the fluid sweep; 1: magnetFlux(X=1, I=[2 3]) (order +1); 2:
     // magnetFlux(X=1, I=[3 2]) (order -1).  One call site per body (they are large).
     for (int step = 0; step < 4; ++step) {
         if (step == 0 || step == 3) {
-            fluid_lean_body<T, LANE1D_BS, KC, true, 0>(a.fa, 0, s_fluid);
+            fluid_lean_body<T, LANE1D_BS, KC, true, 0>(a.fa, 0, s_fluid, dt);
         } else {
             for (int j = 0; j < 2; ++j) {
-                mag_flow_body<T, 0, true>(a.ml[step - 1], j, 0, s_mag);
+                mag_flow_body<T, 0, true>(a.ml[step - 1], j, 0, s_mag, dt);
                 __syncthreads();
             }
-            mag_ct_body<T, 0, true>(a.ml[step - 1], 0, s_mag);
+            mag_ct_body<T, 0, true>(a.ml[step - 1], 0, s_mag, dt);
         }
         __syncthreads();
     }

@@ -146,9 +146,8 @@ struct Tile {
 // The advection of component I[comp] (relaxingMagnet.m:15-50) along D on one tile.
 template <typename T, int D, bool TRK>
 __device__ __forceinline__ void mag_flow_body(const MagnetLeanArgs<T>& ap, int comp,
-                                              long long tile, T* lds) {
+                                              long long tile, T* lds, double dt) {
     const MagnetLeanArgs<T> a = uniform_load(&ap);
-    if (!a.force && !uniform_load(&a.sim->active)) return;
     constexpr bool XM = D == 0;
     constexpr int CH = mlean::CH;
     const int PX = a.PX;
@@ -226,7 +225,6 @@ __device__ __forceinline__ void mag_flow_body(const MagnetLeanArgs<T>& ap, int c
     __syncthreads();
     if (!t.ok) return;  // no barrier follows in this body
 
-    const double dt = uniform_load(&a.sim->dt);
     const double ff = 0.5 * dt / a.dxX;       // relaxingMagnet.m:15
     const T hf = T(ff), hf2 = T(2.0 * ff);    // relaxingMagnet.m:32
     const int nch = (N + CH - 1) / CH;
@@ -350,9 +348,9 @@ __device__ __forceinline__ void mag_flow_body(const MagnetLeanArgs<T>& ap, int c
 // flux.shift(I,1); flux = flux.shift(X,-1); mag(X) = mag(X) - dt/DGRID{I} .* flux), then
 // cellMag_k = 0.5*(B_k + B_k.shift(k,1)) (MagnetArray.m:36-38) of the last component and X.
 template <typename T, int D, bool TRK>
-__device__ __forceinline__ void mag_ct_body(const MagnetLeanArgs<T>& ap, long long tile, T* lds) {
+__device__ __forceinline__ void mag_ct_body(const MagnetLeanArgs<T>& ap, long long tile, T* lds,
+                                            double dt) {
     const MagnetLeanArgs<T> a = uniform_load(&ap);
-    if (!a.force && !uniform_load(&a.sim->active)) return;
     constexpr bool XM = D == 0;
     const int PX = a.PX;
     const mlean::Tile<XM> t(a, D, PX, a.TL, tile);
@@ -362,7 +360,6 @@ __device__ __forceinline__ void mag_ct_body(const MagnetLeanArgs<T>& ap, long lo
     const int mlo = mode_at(a.modes, 0, D), mhi = mode_at(a.modes, 1, D);
     T* const row = lds + (XM ? t.px * N : t.px);
     const int rs = XM ? 1 : PX;
-    const double dt = uniform_load(&a.sim->dt);
 
     // G = F - shift_I(F,+1): flux object, component I == DIRECT (flips for mirror / flip),
     // type 'flux' (zero mode: ghost 0)

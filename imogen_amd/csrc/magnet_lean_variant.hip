@@ -36,8 +36,11 @@ magnet_lean_kernel(const MagnetLeanArgs<T>* args, const BatchTile* tiles, int nt
             if (r > 0 || (int)blockIdx.x >= ntiles) break;
             tile = xcd_tile(blockIdx.x, ntiles);
         }
-        if constexpr (FLOW) mag_flow_body<T, D, TRK>(args[arg], int(tile & 1), tile >> 1, lds);
-        else mag_ct_body<T, D, TRK>(args[arg], tile, lds);
+        double dt;
+        if (sweep_runs(args[arg], dt)) {
+            if constexpr (FLOW) mag_flow_body<T, D, TRK>(args[arg], int(tile & 1), tile >> 1, lds, dt);
+            else mag_ct_body<T, D, TRK>(args[arg], tile, lds, dt);
+        }
         __syncthreads();
     }
 }
