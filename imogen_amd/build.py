@@ -25,7 +25,7 @@ COMMON = [
 ]
 
 SOURCES = ["magnet_dispatch.hip", "cfl.hip", "fluid_dispatch.cpp", "fluid_column.hip",
-           "initial.hip", "source.hip", "imh_api.cpp", "batch.cpp", "serve.cpp", "noalloc.hip",
+           "initial.hip", "source.hip", "imh_api.cpp", "batch.cpp", "download.cpp", "serve.cpp", "noalloc.hip",
            "lane1d.hip", "fluid_long.hip"]
 FP32_ONLY = ("lane1d.hip",)
 VARIANT_SRC = "fluid_sweep_variant.hip"

@@ -287,6 +287,7 @@ static void ctx_free(imh_ctx* c) {
     if (c->sim_ptr) hipFree(c->sim_ptr);
     if (c->par_ptr) hipFree(c->par_ptr);
     if (c->fade_dev) hipFree(c->fade_dev);
+    download_ring_free(c->dl_ring);
     if (c->csum_part) hipFree(c->csum_part);
     if (c->csum_out) hipFree(c->csum_out);
     if (c->long_scratch) hipFree(c->long_scratch);
@@ -865,6 +866,9 @@ extern "C" int imh_download_field(imh_ctx* c, int field, double* out, size_t n) 
     if ((long long)n != c->ncell) return fail(IMH_EINVAL, "array length mismatch");
     hipError_t e = hipStreamSynchronize(c->st);
     if (e != hipSuccess) return hip_fail(e, "stream sync");
+    bool staged;
+    e = download_staged(c, c->f[field], n, esize(c), out, staged);
+    if (staged) return e == hipSuccess ? IMH_OK : hip_fail(e, "download");
     if (c->cfg.precision == IMH_FP64) {
         e = hipMemcpy(out, c->f[field], sizeof(double) * n, hipMemcpyDeviceToHost);
     } else {

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -52,6 +53,11 @@ bool fluid_variant_exists(int esz, int bs, int kmax);
 MagTile choose_mag_tile(int N);
 int column_possible(const imh_config* cfg, int d);
 
+struct DownloadRing;
+void download_ring_free(DownloadRing* r);
+hipError_t download_staged(imh_ctx* c, const void* src, size_t n, size_t esz, double* out,
+                           bool& staged);
+
 }  // namespace imh
 
 struct imh_ctx {
@@ -79,6 +85,8 @@ struct imh_ctx {
     imh::SimDev** sim_ptr = nullptr;        // device array {sim}
     imh::SimParams** par_ptr = nullptr;     // device array {par}
     imh::SimParams host_par;
+    imh::DownloadRing* dl_ring = nullptr;   // download.cpp, under dl_mutex
+    std::mutex dl_mutex;
     double* csum_part = nullptr;
     double* csum_out = nullptr;
     bool obj_init[imh::NOBJ] = {};
