@@ -627,7 +627,9 @@ static hipError_t run_launch(imh_batch* b, const Launch& L, hipStream_t st) {
     const int nb = ((std::max(1, std::min(L.ntiles, b->ncu * 4)) + 7) / 8) * 8;
     switch (L.kind) {
     case L_CFL:
-        return launch_cfl<T>((const CflArgs<T>*)b->cflargs, tl, L.ntiles, nb,
+        // 8 blocks per CU: an ensemble's tiles (most of them a few cells) in one round
+        return launch_cfl<T>((const CflArgs<T>*)b->cflargs, tl, L.ntiles,
+                             ((std::max(1, std::min(L.ntiles, b->ncu * 8)) + 7) / 8) * 8,
                              L.step == 1 ? CFL_RUNNING : CFL_ACTIVE, L.step, 1, st);
     case L_CFL_FINISH:
         return launch_cfl_finish<T>((const CflArgs<T>*)b->cflargs, n,
