@@ -194,13 +194,15 @@ FluidTile choose_fluid_tile(int N, int d, int esz, const TileOverride* ov) {
 // per thread 1 / 2 / 4, 256-thread blocks): FP64 hydro 64x64: 7.7 / 9.7 / -, 48^3: 15.0 /
 // 16.3 / 22.1, 64^3: 22.7 / 19.2 / 24.6, 96^3: 65.9 / 47.9 / 50.4, 200^3: 525 / 362 / 292;
 // FP64 MHD 256x256: 8.6 / 11.2 / 16.5, 100^3 y: 55 / 41 / 43, 150^3 x and z: 210 / 146 /
-// 156 and 289 / 197 / 187, 256^3 z: 1706 / 1148 / 1031; FP32 hydro (2 / 4) 64^3: 14.4 /
-// 15.9, 140^3 x: 94 / 82, 192^3 x: 166 / 140; FP32 MHD 128^3 x and z: 29.5 / 31.7 and 36.2
-// / 32.2, 160^3 z: 119 / 80. Blocks of 256 / 512 threads (FP32, 4 cells): 140^3 z 77.6 /
-// 78.8, 192^3 y and z 137 / 139 and 177 / 150, 256^3 y and z 307 / 287 and 459 / 305, MHD
-// 256^3 y and z 505 / 426 and 664 / 457. Blocks of 256 / 512 / 1024 threads on y pencils:
-// FP64 1024^2: 84.6 / 46.0 / -, FP32 1024^2: 50.4 / 32.8 / 27.7, FP64 512^2: 23.3 / 19.9 /
-// -. 3-D y and z sweeps with rows of 2 / 4 / 8 pencils: FP64 512^3 y 5642 / 7465 / 6406, z
+// 156 and 289 / 197 / 187, 256^3 z: 1706 / 1148 / 1031; FP32 (1 / 2) MHD 191x191 x and y:
+// 6.8 / 9.1 and 9.2 / 10.4, hydro 256x256 x: 6.6 / 8.2, 48^3: 11.7 / 13.4, 64^3: 14.0 /
+// 15.3, y of 512x512 (2 / 4 in 512-thread blocks): 14.8 / 15.9; FP32 hydro (2 / 4) 140^3
+// x: 94 / 82, 192^3 x: 166 / 140; FP32 MHD 128^3 x and z: 29.5 / 31.7 and 36.2 / 32.2,
+// 160^3 z: 119 / 80. Blocks of 256 / 512 threads (FP32, 4 cells): 140^3 z 77.6 / 78.8,
+// 192^3 y and z 137 / 139 and 177 / 150, 256^3 y and z 307 / 287 and 459 / 305, MHD 256^3
+// y and z 505 / 426 and 664 / 457. Blocks of 256 / 512 / 1024 threads on y pencils: FP64
+// 1024^2: 84.6 / 46.0 / -, FP32 1024^2: 50.4 / 32.8 / 27.7, FP64 512^2: 23.3 / 19.9 / -.
+// 3-D y and z sweeps with rows of 2 / 4 / 8 pencils: FP64 512^3 y 5642 / 7465 / 6406, z
 // 10897 / 10498 / 7707, 320^3 z 2533 / 2893 / 2229; FP32 512^3 y 4379 / 2935 / 3335, z
 // 10928 / 5614 / 4147. Past 1024 cells, rows of 1 / 2 pencils in a 3-D grid (32 x 2048 x
 // 2048): FP64 12433 / 8512, FP32 8881 / 5128.
@@ -226,11 +228,11 @@ FluidTile choose_lean_tile(int N, int d, int esz, long long ncell, bool mhd) {
     } else {
         const bool many = ncell > (mhd ? (1 << 22) : (1 << 19));
         if (N <= 256) {
-            ov.kmax = (mhd ? !x && ncell > (3 << 19) : many) ? 4 : 2;
+            ov.kmax = ncell <= (1 << 18) ? 1 : ((mhd ? !x && ncell > (3 << 19) : many) ? 4 : 2);
             if (!x && ncell > (mhd || d == 2 ? (1 << 22) : (1 << 23))) ov.bs = 512;
         } else if (N <= 512) {
             ov.bs = x ? 256 : (d == 2 && many ? 1024 : 512);
-            ov.kmax = (x && !many) ? 2 : 4;
+            ov.kmax = many ? 4 : 2;
         } else {
             ov.bs = x ? (N <= 1024 ? 256 : (N <= 2048 ? 512 : 1024)) : 1024;
             ov.kmax = 4;

@@ -166,11 +166,12 @@ inline bool fluid_needs_general(const FluidArgs<T>& a) {
 
 // Compiled fluid sweep variants X(element size, block size, KMAX): FP64 keeps K <= KMAX
 // cells per thread in registers with KMAX 1..4 (8 for pencils of 2049..4096 cells, with
-// register spills), FP32 with 2..8.  Pencils up to BS * KMAX cells fit one block.  Each
+// register spills), FP32 with 1..8.  Pencils up to BS * KMAX cells fit one block.  Each
 // variant is its own translation unit.
 #define IMH_FLUID_VARIANTS(X) \
     X(8, 256, 1) X(8, 256, 2) X(8, 256, 4) X(8, 512, 2) X(8, 512, 4) X(8, 512, 8) \
-    X(4, 256, 2) X(4, 256, 4) X(4, 512, 4) X(4, 512, 8) X(4, 1024, 4)
+    X(4, 256, 2) X(4, 256, 4) X(4, 512, 4) X(4, 512, 8) X(4, 1024, 4) \
+    X(4, 256, 1) X(4, 512, 2)
 #define IMH_FLUID_LAUNCHER_(E, B, K) launch_fluid_v##E##_##B##_##K
 #define IMH_FLUID_LAUNCHER(E, B, K) IMH_FLUID_LAUNCHER_(E, B, K)
 #define IMH_FLUID_DECLARE(E, B, K)                                                         \
