@@ -145,7 +145,8 @@ def trace_summary(trace_csv, bench_log):
     n = out["roofline"]["launches"]
     fl = [i for i, r in enumerate(rows) if is_fluid(r, "float")][-n:]
     lo, hi = fl[0], fl[-1] + 1
-    while lo > 0 and "begin_iteration" not in rows[lo]["Kernel_Name"]:
+    # the first launch of a step (the time update; a begin launch in older traces)
+    while lo > 0 and not any(k in rows[lo]["Kernel_Name"] for k in ("begin_iteration", "cfl_kernel")):
         lo -= 1
     while hi < len(rows) and "<double" not in rows[hi]["Kernel_Name"] \
             and "copy_probe" not in rows[hi]["Kernel_Name"] and not is_fluid(rows[hi], "float"):
