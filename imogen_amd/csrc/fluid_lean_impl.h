@@ -28,7 +28,7 @@
 //    of the next chunk through two more LDS rows; FP64 96^3 with gravity and radiation 123 -> 43
 //    against the general form).
 // Measured against the general form (us per sweep, mean of the directions): FP64 125^3 175 ->
-// 78, 256^3 1463 -> 621 (1.34 GB: 2.2 TB/s), 333x333 19 -> 15, FP32 192^3 372 -> 147,
+// 75, 256^3 1463 -> 594 (1.34 GB: 2.3 TB/s), 333x333 19 -> 15, FP32 192^3 372 -> 144,
 // 1024x1024 37 -> 26, FP64 MHD 96^3 61 -> 43.  Spilling registers for one more wave per SIMD
 // loses (FP64, 2 cells per thread at 4 waves: 782 -> 1130 at 256^3).
 // Every expression keeps the .m evaluation order (FP64: bit for bit the general form; FP32
@@ -259,12 +259,12 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     constexpr int X = D + 1;
     constexpr int NW = BS / 64;
     constexpr int RL = lean::row_len(BS);
-    // U^n kept in registers where it is cheap; else read again (from the cache) at the end
-#ifdef IMH_LEAN_KEEP
-    constexpr bool KEEP = IMH_LEAN_KEEP;
-#else
-    constexpr bool KEEP = int(sizeof(T)) * K <= 16;
-#endif
+    // Fields whose U^n stays in registers (the others' is read again at the end, mostly past L2:
+    // at FP64 256^3 1275 MB fetched per sweep for 671): all where that is cheap; with four FP64
+    // cells per thread the three that still fit 168 registers (256^3 619 -> 594 us, 200^3 349 ->
+    // 333, 125^3 78 -> 75), which MHD sweeps do not (200^3 358 -> 383).
+    constexpr int KEEP = int(sizeof(T)) * K <= 16 ? 5
+                         : (sizeof(T) == 8 && K == 4 && !MHD && FORM != LEAN_VISC ? 3 : 0);
 
     // not loop-invariant: in a loop over tiles the compiler would keep what follows from it
     // in registers over the whole body
@@ -370,7 +370,7 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     }
 
     // ---- load the chunk (clamped at the pencil end: no branches) ----------------------
-    T q[5][K], bm[3][K], un0[KEEP ? 5 : 1][K];
+    T q[5][K], bm[3][K], un0[KEEP ? KEEP : 1][K];
     if (vec) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) chunk_load<T, K>(a.q[v] + cb(), q[v]);
@@ -392,7 +392,7 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     }
     if constexpr (KEEP) {
 #pragma unroll
-        for (int v = 0; v < 5; ++v)
+        for (int v = 0; v < KEEP; ++v)
 #pragma unroll
             for (int k = 0; k < K; ++k) un0[v][k] = q[v][k];
     }
@@ -759,9 +759,9 @@ __device__ __forceinline__ void fluid_lean_body(const FluidArgs<T>& ap, long lon
     for (int v = 0; v < 5; ++v) {
         __builtin_amdgcn_sched_barrier(0);
         T un[K];
-        if constexpr (KEEP) {
+        if (v < KEEP) {
 #pragma unroll
-            for (int k = 0; k < K; ++k) un[k] = un0[v][k];
+            for (int k = 0; k < K; ++k) un[k] = un0[v < KEEP ? v : 0][k];
         } else if (vec) {
             chunk_load<T, K>(a.q[v] + cb(), un);
         } else {
