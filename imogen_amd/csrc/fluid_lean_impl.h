@@ -80,8 +80,12 @@ struct LMath<double> {
     }
     // x / y with r = rcp(y): the quotient x*r, corrected by its remainder (Markstein's
     // scheme), is the correctly rounded x / y while no intermediate leaves the normal
-    // range (|x| above 1e-290 or zero, y and the quotient within 1e+-290); zeros,
-    // infinities and NaN go through div_fixup.
+    // range (|x| above 1e-290 or zero, y and the quotient within 1e+-290); below it the
+    // remainder underflows and the last bit may be off.  Zeros, infinities and NaN go
+    // through div_fixup; a nonzero x over a subnormal y, or a quotient past the largest
+    // value, is no caller's: they divide by densities (above 1.5e-154, so that the square is
+    // normal), speeds, sums of two differences whose product is x (subnormal only where x is
+    // 0) and the differences that end_ghost lets through.
     static __device__ __forceinline__ double div(double x, double y, double r) {
         const double q = x * r;
         const double e = fma(-y, q, x);
@@ -91,9 +95,9 @@ struct LMath<double> {
     static __device__ __forceinline__ double divrho2(double x, double rho, double r) {
         return div(x, rho, r);
     }
-    // sqrt(x), x >= 0: hardware estimate of 1/sqrt and Newton steps on the root with its exact
-    // remainder (correctly rounded as sqrt() is, without the scaling that only x below
-    // 1e-230 needs).
+    // sqrt(x), x >= 0: hardware estimate of 1/sqrt, Goldschmidt's coupled iteration for the
+    // root and half its reciprocal, and two steps on the root with its exact remainder
+    // (correctly rounded as sqrt() is, without the scaling that only x below 1e-230 needs).
     static __device__ __forceinline__ double root(double x) {
         const double y = __builtin_amdgcn_rsq(x);
         double q = x * y, h = 0.5 * y;
@@ -213,7 +217,12 @@ __device__ __forceinline__ void pin_s(int& x) { asm volatile("" : "+s"(x)); }
 // next.  neg: the shifted component is the shift's direction; zero: zero_shift's
 // ghost of this flux object is 0.  At a transparent end the cubic's argument, 4, lies
 // between its nodes 3 and bcInfinity, and the slope at the far node is 0 (the stored edge
-// repeats there), so one interval's coefficients, from two cells and the edge, suffice; bcInfinity = 4 is that node.
+// repeats there), so one interval's coefficients, from two cells and the edge, suffice;
+// bcInfinity = 4 is that node.
+// Where a difference next to the third node is below 2^-930 (ahead of a front whole rows of
+// cells differ by less than 2e-307), the slope there is taken as 0: its quotients would leave
+// the range of LMath<double>::div, and a slope of that size changes no ghost, as one within
+// 1e-4 of the end cell is that cell.
 __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, double c0, double c1,
                                             int active, int bc_inf, double& tracker) {
     if (mode == IMH_BC_TRANS) {
@@ -225,8 +234,9 @@ __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, doubl
             const double h = double(bc_inf) - 3.0;
             const double rh = LMath<double>::rcp(h);
             const double e1 = c0 - c1, e2 = LMath<double>::div(ev - c0, h, rh);
+            constexpr double TINY = 0x1p-930;
             double d = 0.0;
-            if ((e1 > 0.0 && e2 > 0.0) || (e1 < 0.0 && e2 < 0.0)) {
+            if ((e1 > TINY && e2 > TINY) || (e1 < -TINY && e2 < -TINY)) {
                 const double w1 = 2.0 * h + 1.0, w2 = h + 2.0;
                 d = LMath<double>::quot(w1 + w2, LMath<double>::quot(w1, e1) + LMath<double>::quot(w2, e2));
             }
