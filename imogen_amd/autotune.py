@@ -43,12 +43,14 @@ def sweep_classes(ini, precision):
 
 
 def candidates(n, esz, column_ok, npencil=1 << 30):
-    """Tiles (bs, kmax, px) that hold pencils of n cells with at most half padding."""
+    """Tiles (bs, kmax, px) that hold pencils of n cells with at most half padding.  At most
+    16 pencils per tile: the lean sweep's bound (LEAN_PXMAX); a wider tile would time, and
+    pin the sweep to, the general kernel."""
     out = []
     for e, bs, k in _build.fluid_variants():
         if e != esz:
             continue
-        for px in (1, 2, 4, 8, 16, 32):
+        for px in (1, 2, 4, 8, 16):
             if bs % px:
                 continue
             tl = bs // px
@@ -69,9 +71,10 @@ def load_table(path=TABLE):
 
 
 def tune(sims, precision="fp32", copies_cells=2_000_000, steps=2, table=None, log=None,
-         max_candidates=12):
+         max_candidates=None):
     """Time the candidates of every sweep class of `sims` (a list of (ini, state)) that
-    the table lacks; returns the updated table {class: [bs, kmax, px, us]}."""
+    the table lacks; returns the updated table {class: [bs, kmax, px, us]}.
+    max_candidates: time only the first so many of a class (None: all)."""
     table = dict(table or {})
     esz = 8 if precision == "fp64" else 4
     reps = {}
