@@ -58,6 +58,22 @@ static DownloadRing* download_ring(imh_ctx* c) {
     return c->dl_ring = r;
 }
 
+// The calling thread's current device while an object lives: events belong to the device that
+// is current when they are made, and are recorded on that device's streams only.
+namespace {
+struct OnDevice {
+    int before = -1;
+    explicit OnDevice(int device) {
+        if (hipGetDevice(&before) != hipSuccess || before == device ||
+            hipSetDevice(device) != hipSuccess)
+            before = -1;
+    }
+    ~OnDevice() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
+}  // namespace
+
 // n elements of esz bytes (4: float) at src into out, on the context's stream, which is idle.
 // `staged` is false when the copy is left to the caller: a small field, or no pinned memory.
 hipError_t download_staged(imh_ctx* c, const void* src, size_t n, size_t esz, double* out,
@@ -66,6 +82,7 @@ hipError_t download_staged(imh_ctx* c, const void* src, size_t n, size_t esz, do
     const size_t bytes = n * esz;
     if (bytes < DL_MIN) return hipSuccess;
     std::lock_guard<std::mutex> lock(c->dl_mutex);
+    const OnDevice on(c->cfg.device);
     DownloadRing* r = download_ring(c);
     if (!r) return hipSuccess;
     staged = true;
