@@ -26,35 +26,59 @@ constexpr int DL_THREADS = 4;
 constexpr int DL_RING = 2 * DL_THREADS;  // buffer k % DL_RING belongs to thread k % DL_THREADS
 // below, one chunk's copy costs less than the threads and events
 constexpr size_t DL_MIN = 256 << 10;
+constexpr int DL_DEVICES = 64;
 
 }  // namespace
 
-// The pinned ring of a context, made at its first large download.
+// The pinned ring of a device: made at the first large download from it, shared by its contexts
+// (one download at a time: four threads move a ring's chunks at the pace of the bus), given
+// back with the last context that has used it.
 struct DownloadRing {
+    int device = 0;
+    int users = 0;               // contexts that hold it, under g_rings_mutex
+    std::mutex busy;             // one download at a time
     char* buf = nullptr;
     hipEvent_t ev[DL_RING] = {};
 };
 
-void download_ring_free(DownloadRing* r) {
-    if (!r) return;
+static std::mutex g_rings_mutex;
+static DownloadRing* g_rings[DL_DEVICES];
+
+static void ring_free(DownloadRing* r) {
     for (hipEvent_t& e : r->ev)
         if (e) (void)hipEventDestroy(e);
     if (r->buf) (void)hipHostFree(r->buf);
     delete r;
 }
 
+void download_ring_release(DownloadRing* r) {
+    if (!r) return;
+    std::lock_guard<std::mutex> lock(g_rings_mutex);
+    if (--r->users > 0) return;
+    g_rings[r->device] = nullptr;
+    ring_free(r);
+}
+
+// The ring of the context's device, which is current; nullptr: no pinned memory.
 static DownloadRing* download_ring(imh_ctx* c) {
+    std::lock_guard<std::mutex> lock(g_rings_mutex);
     if (c->dl_ring) return c->dl_ring;
-    DownloadRing* r = new (std::nothrow) DownloadRing();
-    if (!r) return nullptr;
-    hipError_t e = hipHostMalloc((void**)&r->buf, DL_CHUNK * DL_RING, hipHostMallocDefault);
-    for (int i = 0; i < DL_RING && e == hipSuccess; ++i)
-        e = hipEventCreateWithFlags(&r->ev[i], hipEventDisableTiming);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        download_ring_free(r);
-        return nullptr;
+    if (c->cfg.device < 0 || c->cfg.device >= DL_DEVICES) return nullptr;
+    DownloadRing*& r = g_rings[c->cfg.device];
+    if (!r) {
+        r = new (std::nothrow) DownloadRing();
+        hipError_t e = r ? hipHostMalloc((void**)&r->buf, DL_CHUNK * DL_RING, hipHostMallocDefault)
+                         : hipErrorOutOfMemory;
+        for (int i = 0; i < DL_RING && e == hipSuccess; ++i)
+            e = hipEventCreateWithFlags(&r->ev[i], hipEventDisableTiming);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            if (r) ring_free(r);
+            return r = nullptr;
+        }
+        r->device = c->cfg.device;
     }
+    r->users += 1;
     return c->dl_ring = r;
 }
 
@@ -81,10 +105,10 @@ hipError_t download_staged(imh_ctx* c, const void* src, size_t n, size_t esz, do
     staged = false;
     const size_t bytes = n * esz;
     if (bytes < DL_MIN) return hipSuccess;
-    std::lock_guard<std::mutex> lock(c->dl_mutex);
     const OnDevice on(c->cfg.device);
     DownloadRing* r = download_ring(c);
     if (!r) return hipSuccess;
+    std::lock_guard<std::mutex> lock(r->busy);
     staged = true;
     const int nchunk = int((bytes + DL_CHUNK - 1) / DL_CHUNK);
     auto issue = [&](int k) -> hipError_t {

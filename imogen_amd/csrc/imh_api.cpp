@@ -291,7 +291,7 @@ static void ctx_free(imh_ctx* c) {
     if (c->sim_ptr) hipFree(c->sim_ptr);
     if (c->par_ptr) hipFree(c->par_ptr);
     if (c->fade_dev) hipFree(c->fade_dev);
-    download_ring_free(c->dl_ring);
+    download_ring_release(c->dl_ring);
     if (c->csum_part) hipFree(c->csum_part);
     if (c->csum_out) hipFree(c->csum_out);
     if (c->long_scratch) hipFree(c->long_scratch);
@@ -669,6 +669,7 @@ int imh_ctx_recycle(imh_ctx* old, const imh_config* cfg_in, imh_ctx** out) {
     IMH_MOVE(par)
     IMH_MOVE(sim_ptr)
     IMH_MOVE(par_ptr)
+    IMH_MOVE(dl_ring)
     IMH_MOVE(csum_part)
     IMH_MOVE(csum_out)
     IMH_MOVE(arg_host)

@@ -3,7 +3,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -54,7 +53,7 @@ MagTile choose_mag_tile(int N);
 int column_possible(const imh_config* cfg, int d);
 
 struct DownloadRing;
-void download_ring_free(DownloadRing* r);
+void download_ring_release(DownloadRing* r);
 hipError_t download_staged(imh_ctx* c, const void* src, size_t n, size_t esz, double* out,
                            bool& staged);
 
@@ -85,8 +84,7 @@ struct imh_ctx {
     imh::SimDev** sim_ptr = nullptr;        // device array {sim}
     imh::SimParams** par_ptr = nullptr;     // device array {par}
     imh::SimParams host_par;
-    imh::DownloadRing* dl_ring = nullptr;   // download.cpp, under dl_mutex
-    std::mutex dl_mutex;
+    imh::DownloadRing* dl_ring = nullptr;   // download.cpp: the device's, once used
     double* csum_part = nullptr;
     double* csum_out = nullptr;
     bool obj_init[imh::NOBJ] = {};
