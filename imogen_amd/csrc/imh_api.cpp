@@ -422,15 +422,41 @@ static void layout_edges(imh_ctx* c) { c->edges_len = (size_t)edges_layout(c->cf
 
 // Partial sums of the conservation totals (8 fields); the CFL maxima of the tiles follow.
 constexpr size_t CSUM_PART = 2 * 1024 * 8;
+static size_t cfl_part(long long ncell) {
+    const long long chunk = cfl_chunk(ncell);
+    return chunk < ncell ? size_t(3 * ((ncell + chunk - 1) / chunk)) : 0;
+}
+
+// Whether the ends of a configuration let magnetFlux(dX, .) take the lean form: pencils that
+// its windows fit, no fade or wormhole end, and along X both ends circular or neither (a
+// window past a circular end recomputes the other end's cells, which must not depend on
+// ghosts of another mode).
+static bool magnet_lean_ends(const imh_config& g, int dX) {
+    const int ndims = g.grid[2] > 1 ? 3 : 2;
+    if (g.grid[dX] < 8 || g.grid[dX] > MAG_PENCIL_MAX) return false;
+    for (int d = 0; d < 3; ++d)
+        for (int s = 0; s < 2 && (d == dX || d < ndims); ++s)
+            if (g.bc[s][d] == IMH_BC_FADE || g.bc[s][d] == IMH_BC_WORMHOLE) return false;
+    return (g.bc[0][dX] == IMH_BC_CIRC) == (g.bc[1][dX] == IMH_BC_CIRC);
+}
+
+// Scratch fields of the magnetic sweeps: the lean form keeps the limited fluxes of both
+// components (one field more than the general form, which takes them one after the other).
+static int magnet_scratch(const imh_config& g) {
+    if (!g.magnet_active) return 0;
+    for (int d = 0; d < 3; ++d)
+        if (magnet_lean_ends(g, d)) return 2;
+    return 1;
+}
 
 // Device bytes of a context (fields, CT scratch, edge stores, small bookkeeping).
-static size_t ctx_bytes(const imh_config& cfg, size_t edges_len) {
+static size_t ctx_bytes(const imh_config& cfg, size_t edges_len, int scratch_fields) {
     const size_t es = cfg.precision == IMH_FP64 ? 8 : 4;
     const size_t ncell = (size_t)cfg.grid[0] * cfg.grid[1] * cfg.grid[2];
-    size_t b = ncell * es * (IMH_NFIELDS + (cfg.magnet_active ? 2 : 0));
+    size_t b = ncell * es * (IMH_NFIELDS + scratch_fields);
     b += edges_len * sizeof(double) + sizeof(long long) * NOBJ * 6 + 2 * sizeof(SimDev);
-    b += ARG_SLOT * ARG_RING + 6 * ARG_SLOT * CAP_SLOTS + sizeof(double) * (CSUM_PART + 3 * CFL_TILES + 8) +
-         sizeof(double) * MAX_FADE;
+    b += ARG_SLOT * ARG_RING + 6 * ARG_SLOT * CAP_SLOTS +
+         sizeof(double) * (CSUM_PART + cfl_part((long long)ncell) + 8) + sizeof(double) * MAX_FADE;
     return b;
 }
 
@@ -475,13 +501,14 @@ static int ctx_init_host(imh_ctx* c, const imh_config* cfg, bool squeezed) {
                                                : hip_fail(_e, what);                       \
     } while (0)
 
-// Device memory of a context: its stream, the fields, edge stores and bookkeeping.
+// Device memory of a context: its stream, the fields, edge stores and bookkeeping, and
+// last the magnet's scratch_fields (of two only one where the memory does not last: the
+// general magnetic sweep runs on it).
 static int ctx_alloc(imh_ctx* c) {
     const imh_config* cfg = &c->cfg;
     const size_t bytes = (size_t)c->ncell * esize(c);
     CHK(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking), "hipStreamCreate");
     for (int i = 0; i < IMH_NFIELDS; ++i) CHK(hipMalloc(&c->f[i], bytes), "hipMalloc(field)");
-    if (cfg->magnet_active) CHK(hipMalloc(&c->scratch, 2 * bytes), "hipMalloc(scratch)");
     c->edges_cap = c->edges_len;
     CHK(hipMalloc(&c->edges, c->edges_cap * sizeof(double)), "hipMalloc(edges)");
     CHK(hipMalloc(&c->eoff_dev, sizeof(c->eoff)), "hipMalloc(eoff)");
@@ -492,12 +519,23 @@ static int ctx_alloc(imh_ctx* c) {
     CHK(hipMalloc(&c->par_ptr, sizeof(SimParams*)), "hipMalloc(par_ptr)");
     CHK(hipMemcpy(c->sim_ptr, &c->sim, sizeof(SimDev*), hipMemcpyHostToDevice), "sim_ptr");
     CHK(hipMemcpy(c->par_ptr, &c->par, sizeof(SimParams*), hipMemcpyHostToDevice), "par_ptr");
-    CHK(hipMalloc(&c->csum_part, sizeof(double) * (CSUM_PART + 3 * CFL_TILES)), "hipMalloc(csum)");
+    CHK(hipMalloc(&c->csum_part, sizeof(double) * (CSUM_PART + cfl_part(c->ncell))), "hipMalloc(csum)");
     CHK(hipMalloc(&c->csum_out, sizeof(double) * 8), "hipMalloc(csum_out)");
     CHK(hipHostMalloc((void**)&c->arg_host, ARG_SLOT * ARG_RING, hipHostMallocDefault),
         "hipHostMalloc(args)");
     CHK(hipMalloc(&c->arg_dev, ARG_SLOT * ARG_RING), "hipMalloc(args)");
     c->cap_host = new char[ARG_SLOT * CAP_SLOTS];
+    if (c->scratch_fields == 2) {
+        const hipError_t e = hipMalloc(&c->scratch, 2 * bytes);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            c->scratch = nullptr;
+            c->scratch_fields = 1;
+        } else {
+            CHK(e, "hipMalloc(scratch)");
+        }
+    }
+    if (c->scratch_fields == 1) CHK(hipMalloc(&c->scratch, bytes), "hipMalloc(scratch)");
     return IMH_OK;
 }
 
@@ -597,9 +635,21 @@ static int ctx_configure(imh_ctx* c) {
 }
 #undef CHK
 
-extern "C" {
+// imh_memory_estimate of a context made with at most `scratch_fields` of magnet scratch.
+int imh_ctx_estimate(const imh_config* cfg, int scratch_fields, size_t* bytes) {
+    if (!cfg || !bytes) return fail(IMH_EINVAL, "null argument");
+    bool squeezed = false;
+    const imh_config sq = squeeze_grid(*cfg, &squeezed);
+    int rc = validate_config(&sq);
+    if (rc) return rc;
+    long long eoff[NOBJ][2][3];
+    *bytes = ctx_bytes(sq, (size_t)edges_layout(sq, eoff),
+                       std::min(scratch_fields, magnet_scratch(sq)));
+    return IMH_OK;
+}
 
-int imh_create(const imh_config* cfg_in, imh_ctx** out) {
+// imh_create with at most `scratch_fields` of magnet scratch.
+int imh_ctx_create(const imh_config* cfg_in, int scratch_fields, imh_ctx** out) {
     if (!cfg_in || !out) return fail(IMH_EINVAL, "null argument");
     *out = nullptr;
     bool squeezed = false;
@@ -610,6 +660,7 @@ int imh_create(const imh_config* cfg_in, imh_ctx** out) {
     hipError_t e = hipSetDevice(cfg->device);
     if (e != hipSuccess) return hip_fail(e, "hipSetDevice");
     imh_ctx* c = new imh_ctx();
+    c->scratch_fields = std::min(scratch_fields, magnet_scratch(*cfg));
     if ((rc = ctx_init_host(c, cfg, squeezed)) || (rc = ctx_alloc(c)) || (rc = ctx_configure(c))) {
         ctx_free(c);
         return rc;
@@ -618,7 +669,9 @@ int imh_create(const imh_config* cfg_in, imh_ctx** out) {
     return IMH_OK;
 }
 
-}  // extern "C"
+extern "C" int imh_create(const imh_config* cfg, imh_ctx** out) {
+    return imh_ctx_create(cfg, 2, out);
+}
 
 // A new context for cfg on the device memory of `old` (a finished context that is no
 // longer used): same cell count, precision, field set (the magnet's scratch) and room
@@ -656,6 +709,7 @@ int imh_ctx_recycle(imh_ctx* old, const imh_config* cfg_in, imh_ctx** out) {
         old->f[i] = nullptr;
     }
     c->scratch = old->scratch;
+    c->scratch_fields = old->scratch_fields;
     old->scratch = nullptr;
     c->edges = old->edges;
     c->edges_cap = old->edges_cap;
@@ -1034,26 +1088,16 @@ void mag_lean_tile(const imh_ctx* c, int d, int* px, int* tl) {
     *tl = MLEAN_BS / p;
 }
 
-// Whether magnetFlux(dX, [I1 I2]) takes the lean form: the flux objects have their edge
-// stores, uniform spacing, windows that fit the pencil, no fade or wormhole end, and along X
-// both ends circular or neither (a window past a circular end recomputes the other end's
-// cells, which must not depend on ghosts of another mode).
+// Whether magnetFlux(dX, [I1 I2]) takes the lean form: its ends (magnet_lean_ends), the
+// flux objects with their edge stores, uniform spacing, scratch for both components.
 bool magnet_lean_ok(const imh_ctx* c, int dX, const int I[2]) {
-    const imh_config& g = c->cfg;
-    const int N = c->n[dX];
-    if (N < 8 || N > MAG_PENCIL_MAX || c->dline_dev[dX]) return false;
-    auto plain = [&](int d) {
-        for (int s = 0; s < 2; ++s)
-            if (g.bc[s][d] == IMH_BC_FADE || g.bc[s][d] == IMH_BC_WORMHOLE) return false;
-        return true;
-    };
-    if (!plain(dX) || (g.bc[0][dX] == IMH_BC_CIRC) != (g.bc[1][dX] == IMH_BC_CIRC)) return false;
+    if (c->scratch_fields < 2 || !magnet_lean_ends(c->cfg, dX) || c->dline_dev[dX]) return false;
     for (int t = 0; t < 2; ++t) {
         const int dI = I[t] - 1, pair = 3 * dI + dX;
         if (!c->obj_init[OBJ_VG + pair] || !c->obj_init[OBJ_MSFR + pair] ||
             !c->obj_init[OBJ_WMAG + pair] || !c->obj_init[OBJ_MFLUX + pair])
             return false;
-        if (dI < c->ndims && (!plain(dI) || c->dline_dev[dI])) return false;
+        if (dI < c->ndims && c->dline_dev[dI]) return false;
     }
     return true;
 }
@@ -1999,19 +2043,12 @@ int imh_conservation_sums(imh_ctx* c, double out[8]) {
 
 int imh_memory_bytes(imh_ctx* c, size_t* bytes) {
     if (!c || !bytes) return fail(IMH_EINVAL, "null argument");
-    *bytes = ctx_bytes(c->cfg, c->edges_len);
+    *bytes = ctx_bytes(c->cfg, c->edges_len, c->cfg.magnet_active ? c->scratch_fields : 0);
     return IMH_OK;
 }
 
 int imh_memory_estimate(const imh_config* cfg, size_t* bytes) {
-    if (!cfg || !bytes) return fail(IMH_EINVAL, "null argument");
-    bool squeezed = false;
-    const imh_config sq = squeeze_grid(*cfg, &squeezed);
-    int rc = validate_config(&sq);
-    if (rc) return rc;
-    long long eoff[NOBJ][2][3];
-    *bytes = ctx_bytes(sq, (size_t)edges_layout(sq, eoff));
-    return IMH_OK;
+    return imh_ctx_estimate(cfg, 2, bytes);
 }
 
 // Tuning hook (used by the autotuner): override the fluid tile of one sweep dim.

@@ -68,7 +68,8 @@ struct imh_ctx {
     int active_lin[3];
     hipStream_t st = nullptr;
     void* f[IMH_NFIELDS] = {};
-    void* scratch = nullptr;        // mag(I).flux(X) for the CT steps, both components
+    void* scratch = nullptr;        // mag(I).flux(X) for the CT steps
+    int scratch_fields = 0;         // 2: of both components (lean magnetic sweep), 1: of one
     double* edges = nullptr;
     size_t edges_len = 0;
     size_t edges_cap = 0;               // doubles allocated at edges (>= edges_len)
@@ -226,4 +227,6 @@ double source_bytes(const imh_ctx* c);
 void imh_ctx_free(imh_ctx* c);
 // A new context for cfg on the device memory of a finished one (same cell count,
 // precision, field set, room for the edge stores); see imh_api.cpp.
+int imh_ctx_create(const imh_config* cfg, int scratch_fields, imh_ctx** out);
+int imh_ctx_estimate(const imh_config* cfg, int scratch_fields, size_t* bytes);
 int imh_ctx_recycle(imh_ctx* old, const imh_config* cfg, imh_ctx** out);

@@ -35,6 +35,7 @@ struct Request {
     int status = IMH_REQ_QUEUED;
     imh_ctx* ctx = nullptr;
     size_t bytes = 0;
+    size_t least = 0;                 // with one field of magnet scratch (general magnetic sweep)
     double t_submit = 0, t_admit = -1, t_done = -1;
     SimDev last{};
 };
@@ -93,12 +94,14 @@ static void release_request(imh_server* s, Request& r) {
 // A context for request r: a pooled one of the same cell count, precision and field set
 // when there is one (its memory reused), else a new one.  Pooled contexts are freed,
 // oldest first, while the budget needs their memory.
-static int context_for(imh_server* s, Request& r) {
+static int context_for(imh_server* s, Request& r, bool least) {
     const long long ncell = (long long)r.n;
+    const int scratch = least || r.bytes == r.least ? 1 : 2;
     for (size_t i = 0; i < s->pool.size(); ++i) {
         imh_ctx* p = s->pool[i].ctx;
         if (p->ncell != ncell || p->cfg.precision != r.cfg.precision ||
-            (r.cfg.magnet_active && !p->cfg.magnet_active))
+            (r.cfg.magnet_active && (!p->cfg.magnet_active || p->scratch_fields < scratch ||
+                                     (least && p->scratch_fields > scratch))))
             continue;
         const size_t pb = s->pool[i].bytes;
         const int rc = imh_ctx_recycle(p, &r.cfg, &r.ctx);
@@ -112,14 +115,16 @@ static int context_for(imh_server* s, Request& r) {
         s->pooled -= std::min(s->pooled, s->pool.front().bytes);
         s->pool.pop_front();
     }
-    return imh_create(&r.cfg, &r.ctx);
+    return imh_ctx_create(&r.cfg, scratch, &r.ctx);
 }
 
 // Admit queued requests in order while a slot is free and the budget allows.
 static int admit(imh_server* s) {
     while (!s->queue.empty() && (int)s->active.size() < s->max_active) {
         Request& r = s->reqs[s->queue.front()];
-        if (s->used + r.bytes > s->budget) {
+        // a magnetic request whose second scratch field is past the budget runs without it
+        const bool least = s->used + r.bytes > s->budget;
+        if (s->used + r.least > s->budget) {
             if (s->active.empty() && s->used == 0) {
                 // can never fit: fail it rather than block the queue forever
                 r.status = IMH_REQ_FAILED;
@@ -131,7 +136,7 @@ static int admit(imh_server* s) {
         }
         const long long id = s->queue.front();
         s->queue.pop_front();
-        int rc = context_for(s, r);
+        int rc = context_for(s, r, least);
         if (rc == IMH_OK && r.ic_kind > 0) {
             rc = imh_init_problem(r.ctx, r.ic_kind, r.ic_params.data(), (int)r.ic_params.size());
         } else if (rc == IMH_OK) {
@@ -152,6 +157,7 @@ static int admit(imh_server* s) {
         r.state.clear();
         r.state.shrink_to_fit();
         r.status = IMH_REQ_RUNNING;
+        (void)imh_memory_bytes(r.ctx, &r.bytes);
         r.t_admit = now_s(s);
         s->used += r.bytes;
         s->active.push_back(id);
@@ -255,8 +261,9 @@ int imh_serve_submit(imh_server* s, const imh_config* cfg, const double* mass,
     imh_config c = *cfg;
     c.precision = s->precision;
     c.device = s->device;
-    size_t bytes = 0;
+    size_t bytes = 0, least = 0;
     int rc = imh_memory_estimate(&c, &bytes);
+    if (!rc) rc = imh_ctx_estimate(&c, 1, &least);
     if (rc) return rc;
     const size_t ncell = (size_t)c.grid[0] * c.grid[1] * c.grid[2];
     if (n != ncell) return fail(IMH_EINVAL, "state has %zu cells, the grid %zu", n, ncell);
@@ -264,6 +271,7 @@ int imh_serve_submit(imh_server* s, const imh_config* cfg, const double* mass,
     r.cfg = c;
     r.n = n;
     r.bytes = bytes;
+    r.least = least;
     r.state.resize(8 * n);
     const double* src[8] = {mass, mom[0], mom[1], mom[2], ener, mag[0], mag[1], mag[2]};
     for (int f = 0; f < 8; ++f) {
@@ -286,13 +294,15 @@ int imh_serve_submit_problem(imh_server* s, const imh_config* cfg, int kind,
     imh_config c = *cfg;
     c.precision = s->precision;
     c.device = s->device;
-    size_t bytes = 0;
+    size_t bytes = 0, least = 0;
     int rc = imh_memory_estimate(&c, &bytes);
+    if (!rc) rc = imh_ctx_estimate(&c, 1, &least);
     if (rc) return rc;
     Request r;
     r.cfg = c;
     r.n = (size_t)c.grid[0] * c.grid[1] * c.grid[2];
     r.bytes = bytes;
+    r.least = least;
     r.ic_kind = kind;
     r.ic_params.assign(params, params + nparams);
     r.t_submit = now_s(s);

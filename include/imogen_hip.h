@@ -212,7 +212,10 @@ int imh_conservation_sums_noalloc(const void *const *fields, int nfields, int pr
 
 /* Device bytes held by the context. */
 int imh_memory_bytes(imh_ctx *ctx, size_t *bytes);
-/* Device bytes a context with this configuration would hold (validates cfg first). */
+/* Device bytes a context with this configuration would hold (validates cfg first).  With an
+ * evolved magnetic field one field of them, the second scratch field of the magnetic sweeps,
+ * can be done without: a context that finds no memory for it runs the slower sweeps that
+ * need one. */
 int imh_memory_estimate(const imh_config *cfg, size_t *bytes);
 
 /* ---- initial conditions on the device ---------------------------------------------------
@@ -300,7 +303,8 @@ int imh_batch_set_viscosity(imh_batch *b, int sim, int type, double linear, doub
 /* ---- serving loop (continuous batching of solve requests on one device) ------------ */
 /* A request is one simulation run while TimeManager.running holds (to its TIMEMAX or
  * ITERMAX).  Requests queue in FIFO order and are admitted while fewer than max_active
- * run and their device memory (imh_memory_estimate) fits the HBM budget; admitted
+ * run and their device memory (imh_memory_estimate; without the second scratch field of the
+ * magnetic sweeps where only that fits) fits the HBM budget; admitted
  * requests stay resident and advance together with the running ones; finished ones leave
  * the batch at the end of the round and keep their result on the device until
  * imh_serve_release.  No counterpart in the reference (its main loop runs one simulation). */
