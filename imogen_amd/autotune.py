@@ -86,6 +86,7 @@ def tune(sims, precision="fp32", copies_cells=2_000_000, steps=2, table=None, lo
         rc = from_ini(ini)
         m = int(max(1, min(64, copies_cells // max(1, rc.ncell))))
         ens = Ensemble([(ini, st)] * m, precision)
+        ens.set_fused_1d(False)  # the 1-D lane has a tile of its own: time the sweep's launches
         ens.step(1)
         best = None
         # tiles that hold every pencil length of the class (rounded up to a power of 2)

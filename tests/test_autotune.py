@@ -9,7 +9,10 @@ class Recorder:
     tiles = []
 
     def __init__(self, sims, precision):
-        pass
+        self.fused = True  # 1-D MHD simulations: one launch, no fluid sweeps
+
+    def set_fused_1d(self, enable):
+        self.fused = bool(enable)
 
     def step(self, n):
         pass
@@ -19,7 +22,7 @@ class Recorder:
             self.tiles.append((X, (bs, k, px)))
 
     def profile_step(self, n):
-        return {"fluid": (1.0, 0.0, 1)}
+        return {"fluid": (0.0, 0.0, 0) if self.fused else (1.0, 0.0, 1)}
 
     def close(self):
         pass
@@ -44,3 +47,11 @@ def test_candidates_take_the_lean_sweep():
     for esz in (4, 8):
         for n in (8, 16, 64, 200, 4096):
             assert all(px <= 16 for bs, k, px in autotune.candidates(n, esz, True, 1 << 20))
+
+
+def test_one_dimensional_sweeps_are_timed(monkeypatch):
+    """1-D MHD simulations run in one launch per iteration, without the sweep that the tile is
+    for; the tuner times that sweep."""
+    monkeypatch.setattr(autotune, "Ensemble", Recorder)
+    table = autotune.tune([problems.mhd_riemann(300, seed=1)], "fp32")
+    assert table and all(us > 0 for _, _, _, us in table.values())
