@@ -587,24 +587,18 @@ PLAIN_SWEEP = "auto_fast"
 
 def large_plain_roofline(args):
     """Plain FP64 path on Sedov 256^3: HIP-event time of every launch over two profiled
-    iterations, with the plain path's sweep and, beside it, with the general sweep."""
+    iterations."""
     import imogen_amd
     from imogen_amd import problems
     ini, st = problems.sedov(256)
-    res = {}
-    # the plain path's sweep last: trace and counter summaries take the last launches
-    for kind in ("general", PLAIN_SWEEP):
-        run = imogen_amd.initialize(ini, "fp64")
-        imogen_amd.create_arrays(run, st)
-        run.set_fluid_kernel(kind)
-        run.run_iterations(1)
-        prof = run.profile_iterations(2)
-        run.close()
-        res[kind] = roofline(prof, "sedov 256^3 hydro FP64, plain path")
-    del st
-    out = res[PLAIN_SWEEP]
-    out["sweep"] = "lean sweep (%s)" % PLAIN_SWEEP
-    out["general_sweep"] = {k: res["general"][k] for k in ("achieved", "frac", "avg_launch_us")}
+    run = imogen_amd.initialize(ini, "fp64")
+    imogen_amd.create_arrays(run, st)
+    run.set_fluid_kernel(PLAIN_SWEEP)
+    run.run_iterations(1)
+    prof = run.profile_iterations(2)
+    run.close()
+    out = roofline(prof, "sedov 256^3 hydro FP64, plain path")
+    out["sweep"] = "lean sweep"
     return out
 
 

@@ -102,8 +102,10 @@ def build(verbose=False, jobs=None, incremental=False, out=None, defines=()):
     unless `incremental` (then only objects older than some source or header).
 
     `out` links the library elsewhere (loaded when IMH_LIB_PATH names it) and `defines`
-    (NAME=VALUE) set the compile-time tuning knobs of the kernels, e.g.
-    IMH_FLUID_WAVES_PER_EU or IMH_FLUID_GROUP (fluid_sweep_impl.h)."""
+    (NAME=VALUE) set the compile-time tuning knobs of the kernels: the waves per SIMD that
+    IMH_LEAN_WAVES (fluid_lean_variant.hip), IMH_MLEAN_WAVES (magnet_lean_variant.hip),
+    IMH_LANE1D_WAVES (lane1d.hip) and IMH_FLUID_WAVES_PER_EU (fluid_sweep_variant.hip)
+    leave registers for."""
     lib_path = os.path.abspath(out) if out else LIB
     build_dir = BUILD if not out else os.path.join(
         BUILD, "alt_" + os.path.splitext(os.path.basename(lib_path))[0])

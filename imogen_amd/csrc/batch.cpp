@@ -84,8 +84,6 @@ struct imh_batch {
     hipStream_t st = nullptr;
     std::vector<imh_ctx*> ctx;
     int ncu = 256;
-    SimDev** sims_dev = nullptr;
-    SimParams** pars_dev = nullptr;
     void* fargs = nullptr;    // FluidArgs<T>[n*3]
     void* margs = nullptr;    // MagnetArgs<T>[n*9], index sim*9 + 3*dI + dX
     void* mlargs = nullptr;   // MagnetLeanArgs<T>[n*6], index sim*6 + mlean_index(dX, I)
@@ -152,8 +150,6 @@ static void batch_free(imh_batch* b) {
     if (!b) return;
     if (b->st) hipStreamSynchronize(b->st);
     free_plans(b);
-    hipFree(b->sims_dev);
-    hipFree(b->pars_dev);
     hipFree(b->fargs);
     hipFree(b->margs);
     hipFree(b->mlargs);
@@ -283,32 +279,20 @@ static int batch_setup(imh_batch* b) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, b->device) == hipSuccess && prop.multiProcessorCount > 0)
         b->ncu = prop.multiProcessorCount;
-    size_t es = b->prec == IMH_FP64 ? 8 : 4;
-    (void)es;
-    hipError_t e = hipMalloc(&b->sims_dev, sizeof(SimDev*) * n);
-    if (e == hipSuccess) e = hipMalloc(&b->pars_dev, sizeof(SimParams*) * n);
     size_t fsz = b->prec == IMH_FP64 ? sizeof(FluidArgs<double>) : sizeof(FluidArgs<float>);
     size_t msz = b->prec == IMH_FP64 ? sizeof(MagnetArgs<double>) : sizeof(MagnetArgs<float>);
     size_t mlsz = b->prec == IMH_FP64 ? sizeof(MagnetLeanArgs<double>) : sizeof(MagnetLeanArgs<float>);
     size_t csz = b->prec == IMH_FP64 ? sizeof(CellMagArgs<double>) : sizeof(CellMagArgs<float>);
     size_t lsz = b->prec == IMH_FP64 ? sizeof(CflArgs<double>) : sizeof(CflArgs<float>);
-    if (e == hipSuccess) e = hipMalloc(&b->fargs, fsz * n * 3);
+    hipError_t e = hipMalloc(&b->fargs, fsz * n * 3);
     if (e == hipSuccess) e = hipMalloc(&b->margs, msz * n * 9);
     if (e == hipSuccess) e = hipMalloc(&b->mlargs, mlsz * n * 6);
     if (e == hipSuccess) e = hipMalloc(&b->cargs, csz * n * 3);
     if (e == hipSuccess) e = hipMalloc(&b->cflargs, lsz * n);
     if (e != hipSuccess) return hip_fail(e, "batch allocation");
-    std::vector<SimDev*> sp(n);
-    std::vector<SimParams*> pp(n);
     b->any_step_mode = false;
-    for (int i = 0; i < n; ++i) {
-        sp[i] = b->ctx[i]->sim;
-        pp[i] = b->ctx[i]->par;
+    for (int i = 0; i < n; ++i)
         if (b->ctx[i]->cfg.update_mode == 0) b->any_step_mode = true;
-    }
-    e = hipMemcpy(b->sims_dev, sp.data(), sizeof(SimDev*) * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(b->pars_dev, pp.data(), sizeof(SimParams*) * n, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return hip_fail(e, "batch pointers");
     return IMH_OK;
 }
 

@@ -43,7 +43,7 @@ enum FluxType : int { FT_OTHER = 0, FT_FLUXL = 1, FT_FLUXR = 2, FT_FLUX = 3 };
 struct SimDev {
     double dt;                 // run.time.dTime
     double time;               // run.time.time
-    double spare[3];
+    double spare[3];           // unused: keeps the layout of saved checkpoints
     int iteration;             // run.time.iteration
     int grid_index;            // last CFL direction
     int error;                 // IMH_ECFL when no speed exceeds 1e-2

@@ -17,9 +17,8 @@
 // the workgroup (LANE1D_BS threads of LANE1D_KMAX, 3/4, 1/2 or 1/4 of it cells each: the
 // bodies are instantiated for all four, sharing their LDS, and a simulation runs the
 // smallest that holds its pencil), so the results are those of the per-launch plan bit for
-// bit.  The time step comes from the batch-wide CFL launch before, the iteration counters
-// from the batch-wide launch after.  The state stays in the workgroup's L2 between the
-// steps.  Bound by the latency of the longest pencils' chain (128 simulations of 256..4096
+// bit.  The time step and the iteration count come from the batch-wide time update before.
+// The state stays in the workgroup's L2 between the steps.  Bound by the latency of the longest pencils' chain (128 simulations of 256..4096
 // cells: 130 us per iteration; 228 with the general fluid and magnet bodies, 181 with the lean
 // fluid body alone); two waves per SIMD, as four (128 registers) spill the 8-cell body.
 #include "fluid_lean_impl.h"
