@@ -82,10 +82,13 @@ struct LMath<double> {
     // scheme), is the correctly rounded x / y while no intermediate leaves the normal
     // range (|x| above 1e-290 or zero, y and the quotient within 1e+-290); below it the
     // remainder underflows and the last bit may be off.  Zeros, infinities and NaN go
-    // through div_fixup; a nonzero x over a subnormal y, or a quotient past the largest
-    // value, is no caller's: they divide by densities (above 1.5e-154, so that the square is
-    // normal), speeds, sums of two differences whose product is x (subnormal only where x is
-    // 0) and the differences that end_ghost lets through.
+    // through div_fixup, and so does a quotient past the largest value: its remainder makes
+    // a NaN of it, which div_fixup takes, over finite operands, for an overflow and returns
+    // as infinity of the right sign (gfx950; so does any x over a y below 5.6e-309, whose
+    // reciprocal overflows: right where the quotient does).  Callers divide by densities
+    // (above 1.5e-154, so that the square is normal), speeds, sums of two differences whose
+    // product is x (subnormal only where x is 0) and, with x of 3 and more, the differences of
+    // end_ghost.
     static __device__ __forceinline__ double div(double x, double y, double r) {
         const double q = x * r;
         const double e = fma(-y, q, x);
@@ -219,10 +222,9 @@ __device__ __forceinline__ void pin_s(int& x) { asm volatile("" : "+s"(x)); }
 // between its nodes 3 and bcInfinity, and the slope at the far node is 0 (the stored edge
 // repeats there), so one interval's coefficients, from two cells and the edge, suffice;
 // bcInfinity = 4 is that node.
-// Where a difference next to the third node is below 2^-930 (ahead of a front whole rows of
-// cells differ by less than 2e-307), the slope there is taken as 0: its quotients would leave
-// the range of LMath<double>::div, and a slope of that size changes no ghost, as one within
-// 1e-4 of the end cell is that cell.
+// Ahead of a front the differences next to the third node fall below 2e-307 in whole rows of
+// cells; the slope's quotients by them overflow to infinity (LMath<double>::div), and the slope
+// is 0, as with divisions.
 __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, double c0, double c1,
                                             int active, int bc_inf, double& tracker) {
     if (mode == IMH_BC_TRANS) {
@@ -234,9 +236,8 @@ __device__ __forceinline__ double end_ghost(int mode, bool neg, bool zero, doubl
             const double h = double(bc_inf) - 3.0;
             const double rh = LMath<double>::rcp(h);
             const double e1 = c0 - c1, e2 = LMath<double>::div(ev - c0, h, rh);
-            constexpr double TINY = 0x1p-930;
             double d = 0.0;
-            if ((e1 > TINY && e2 > TINY) || (e1 < -TINY && e2 < -TINY)) {
+            if ((e1 > 0.0 && e2 > 0.0) || (e1 < 0.0 && e2 < 0.0)) {
                 const double w1 = 2.0 * h + 1.0, w2 = h + 2.0;
                 d = LMath<double>::quot(w1 + w2, LMath<double>::quot(w1, e1) + LMath<double>::quot(w2, e2));
             }
