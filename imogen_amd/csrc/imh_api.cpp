@@ -1089,9 +1089,11 @@ void mag_lean_tile(const imh_ctx* c, int d, int* px, int* tl) {
 }
 
 // Whether magnetFlux(dX, [I1 I2]) takes the lean form: its ends (magnet_lean_ends), the
-// flux objects with their edge stores, uniform spacing, scratch for both components.
+// flux objects with their edge stores, uniform spacing, scratch for both components, and two
+// different ones (a direct call may name one twice: its second advection starts from the
+// first's result, while the lean form advects both at once, in place).
 bool magnet_lean_ok(const imh_ctx* c, int dX, const int I[2]) {
-    if (c->scratch_fields < 2 || !magnet_lean_ends(c->cfg, dX) || c->dline_dev[dX]) return false;
+    if (I[0] == I[1] || c->scratch_fields < 2 || !magnet_lean_ends(c->cfg, dX) || c->dline_dev[dX]) return false;
     for (int t = 0; t < 2; ++t) {
         const int dI = I[t] - 1, pair = 3 * dI + dX;
         if (!c->obj_init[OBJ_VG + pair] || !c->obj_init[OBJ_MSFR + pair] ||
