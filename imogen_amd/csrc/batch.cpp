@@ -302,13 +302,7 @@ static int run_first_iterations(imh_batch* b, bool* changed) {
     *changed = false;
     for (imh_ctx* c : b->ctx) {
         if (!c->have_state) return fail(IMH_ESTATE, "batch simulation without uploaded state");
-        bool fresh = (c->cfg.fluid_active && !c->fluid_init);
-        if (!fresh && c->cfg.magnet_active) {
-            for (int dI = 0; dI < 3 && !fresh; ++dI)
-                for (int dX = 0; dX < 3 && !fresh; ++dX)
-                    if (dI != dX && c->n[dX] >= 3 && !c->obj_init[OBJ_VG + 3 * dI + dX]) fresh = true;
-        }
-        if (!fresh) continue;
+        if (flux_objects_ready(c)) continue;
         hipStream_t own = c->st;
         c->st = b->st;
         int rc = imh_iteration_body(c, 1);

@@ -1362,6 +1362,18 @@ int imh_iteration_body(imh_ctx* c, int conditional) {
     return IMH_OK;
 }
 
+// Whether every flux object of the loop body has its edge stores (its first assignment lies
+// behind): a sweep that still makes them must not be captured, as each replay would make
+// them again.
+bool flux_objects_ready(const imh_ctx* c) {
+    if (c->cfg.fluid_active && !c->fluid_init) return false;
+    if (c->cfg.magnet_active)
+        for (int dI = 0; dI < 3; ++dI)
+            for (int dX = 0; dX < 3; ++dX)
+                if (dI != dX && c->n[dX] >= 3 && !c->obj_init[OBJ_VG + 3 * dI + dX]) return false;
+    return true;
+}
+
 // Whether the loop body of a 1-D simulation can run in the one-workgroup kernel
 // (line1d_variant.hip): lean sweeps only, no source terms, no viscosity.
 static bool line1d_ok(const imh_ctx* c) {
@@ -1637,8 +1649,7 @@ int imh_run(imh_ctx* c, int max_iterations, int* done) {
     const int start = sd.iteration;
     int todo = std::min(max_iterations, c->cfg.iter_max - start + 1);
     for (int it = 0; it < todo; ++it) {
-        bool inited = c->fluid_init || !c->cfg.fluid_active;
-        if (!inited || c->no_graphs) {
+        if (!flux_objects_ready(c) || c->no_graphs) {
             if ((rc = imh_iteration_body(c, 1))) return rc;
         } else if (line1d_ok(c)) {
             // up to the next look at the time state in one launch

@@ -204,6 +204,7 @@ int imh_fluid_sweep_internal(imh_ctx* c, int X, int force);
 int imh_magnet_sweep_internal(imh_ctx* c, int X, const int I[2], int force);
 int imh_time_update_internal(imh_ctx* c, int step, int gate, int count);
 int imh_flux_internal(imh_ctx* c, int order, int force);
+bool flux_objects_ready(const imh_ctx* c);
 
 // argument blocks of one simulation (imh_api.cpp), shared with the batched path
 template <typename T>
